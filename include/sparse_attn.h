@@ -81,14 +81,15 @@ const char* sa_last_error(void);
  *
  * workspace (optional, sa_prefill_workspace_bytes() bytes, 4-byte aligned):
  * with it the kernel runs one persistent workgroup per resident slot that
- * claims work items from counters in the workspace.  It must be zeroed before
+ * takes its first work items by index and claims the others from counters in
+ * the workspace.  It must be zeroed before
  * its first use; every completed launch leaves its counters zeroed again.
  * Launches that may run concurrently (other streams, graph replays on other
  * streams) must not share one workspace: keep one per stream.  Word 3 of the
  * workspace is a status word that launches only set and the caller clears:
- * bit 0 means a launch processed fewer work items than it has (its counters
- * were not zero at launch, or an overlapping launch shared them) and left the
- * skipped items' outputs unwritten.  NULL launches one workgroup per work
+ * bit 0 means a launch's counters were not zero at launch or an overlapping
+ * launch shared them: it may have processed fewer work items than it has and
+ * left the skipped items' outputs unwritten.  NULL launches one workgroup per work
  * item instead.
  */
 int sa_prefill(int dtype,

@@ -31,8 +31,8 @@
 //    32..63 in a wave whose rows all end before them: the lower half on a diagonal tile;
 //  * O is written back through LDS so that every global store is a 16-byte piece of a
 //    contiguous row;
-//  * with a workspace, one persistent workgroup per CU slot claims work items from an
-//    atomic counter, heaviest query tiles first.
+//  * with a workspace, one persistent workgroup per CU slot takes its first work items by its
+//    own index and claims further ones from an atomic counter, heaviest query tiles first.
 //
 // MFMA 32x32x16 lane layouts used (l = lane, g = l / 32):
 //   A (32 x 16): lane l holds row l % 32, k = 8g .. 8g+7
@@ -55,6 +55,8 @@ constexpr int N_XCD = 8;         // XCDs of an MI355X; workgroups are dealt to t
 constexpr int XCD_CHUNK = 4;     // query tiles per chunk dealt to one XCD
 // Largest token stride (elements) of K and V: per-lane offsets within a tile are 32-bit.
 constexpr int64_t MAX_KV_STRIDE = (int64_t)1 << 24;
+
+constexpr int LOOKAHEAD = 3;     // items a four-head workgroup holds before it claims from the counter
 
 struct PrefillArgs {
   const elem_t* q;
@@ -106,10 +108,10 @@ struct PrefillArgs {
 };
 
 // Words of the persistent-launch workspace: the next unclaimed item, the workgroups done, the
-// items processed, and a status word that only the host clears.  A launch whose workgroups
-// processed fewer items than it has (the counters were not zero at launch, or two launches
-// that overlapped in time shared them) sets WS_SKIPPED: the skipped items' outputs are not
-// written, so the caller must not use the output.
+// items processed, and a status word that only the host clears.  A launch that found the counters
+// not zero, or whose workgroups processed another number of items than it has (two launches that
+// overlapped in time shared the counters), sets WS_SKIPPED: items may have been skipped and their
+// outputs not written, so the caller must not use the output.
 enum : int { WS_NEXT = 0, WS_DONE_WG = 1, WS_DONE_ITEMS = 2, WS_STATUS = 3, WS_WORDS = 8 };
 constexpr unsigned WS_SKIPPED = 1u;
 
@@ -905,7 +907,7 @@ struct Prefill {
         ld.o0 = o[0];
         ld.o1 = o[1];
       }
-      ld.nv = atomicAdd(&a.counter[WS_NEXT], 1u);
+      ld.nv = LOOKAHEAD * gridDim.x + atomicAdd(&a.counter[WS_NEXT], 1u);
     }
   }
 
@@ -1327,7 +1329,15 @@ struct Prefill {
       item(a, qt, r, hs, b, sKV, s_row, s_mask);
   }
 
-  // Persistent four-head loop with lookahead.  Item i of this workgroup finds in LDS its id,
+  // Persistent four-head loop with lookahead.  The first LOOKAHEAD items of a workgroup w are fixed
+  // by w, later ones are claimed from the counter.  (Claimed ahead, the first ones all went to the
+  // workgroups that started first, three each: 128 items of 64-79 tiles -- 1,000 queries of 32
+  // heads on 5,000 keys -- ran on 43 CUs, 297 us; one item per workgroup takes 107 us.)  With fewer
+  // items than LOOKAHEAD per workgroup, item w comes first and the second round runs in reverse, so
+  // the workgroup with the lightest first item takes the heaviest second one; with more, w takes
+  // three neighbouring items as a claim would have given it (w, 2g - 1 - w, 2g + w there: prefill of
+  // 32K tokens 332.7 against 330.0 us).
+  // Item i of this workgroup finds in LDS its id,
   // CSR offsets and (qt, r, hs, b) (slot i % 4 of s_meta) and its row (row cache i % 2), and
   // the id, offsets and row of item i + 1 and the id of item i + 2; its prologue fetches the
   // row of item i + 1, the offsets and (qt, r, hs, b) of item i + 2 and claims item i + 3
@@ -1342,12 +1352,11 @@ struct Prefill {
     __shared__ __attribute__((aligned(16))) int s_meta[4][8];
     const int tid = threadIdx.x;
     if (tid == 0) {
-      const unsigned v0 = atomicAdd(&a.counter[WS_NEXT], 1u);
-      const unsigned v1 = atomicAdd(&a.counter[WS_NEXT], 1u);
-      const unsigned v2 = atomicAdd(&a.counter[WS_NEXT], 1u);
-      s_meta[0][0] = (int)v0;
-      s_meta[1][0] = (int)v1;
-      s_meta[2][0] = (int)v2;
+      const int g = (int)gridDim.x, w = (int)blockIdx.x;
+      const bool many = n_items >= LOOKAHEAD * g;
+      s_meta[0][0] = many ? LOOKAHEAD * w : w;
+      s_meta[1][0] = many ? LOOKAHEAD * w + 1 : 2 * g - 1 - w;
+      s_meta[2][0] = many ? LOOKAHEAD * w + 2 : 2 * g + w;
     }
     __syncthreads();
     if (tid < 2) {
@@ -1466,24 +1475,27 @@ struct Prefill {
         if (threadIdx.x < 2 * TL_HALF_WORDS) rec[4 + threadIdx.x] = s_tl[threadIdx.x / TL_HALF_WORDS][threadIdx.x % TL_HALF_WORDS];
       }
     } else {
-      for (;;) {
-        if (threadIdx.x == 0) s_item = (int)atomicAdd(&a.counter[WS_NEXT], 1u);
-        __syncthreads();
-        const int v = s_item;
-        __syncthreads();
-        if (v >= n_items) break;
+      __syncthreads();  // row ranks visible, and the K/V buffers they were computed in free
+      for (int v = (int)blockIdx.x; v < n_items;) {  // the first item is this workgroup's own
         process(a, v, sKV, sQ, s_row, s_mask);
         ++done;
+        if (threadIdx.x == 0) s_item = (int)(gridDim.x + atomicAdd(&a.counter[WS_NEXT], 1u));
+        __syncthreads();
+        v = s_item;
+        __syncthreads();
       }
     }
     // Items processed, then this workgroup done; the last one checks the total and zeroes the
-    // counters for the next launch on the stream.
+    // counters for the next launch on the stream.  Every processed item made one claim, so a
+    // counter that was zero at launch ends at n_items too.
     if (threadIdx.x == 0) {
       atomicAdd(&a.counter[WS_DONE_ITEMS], (unsigned)done);
       __threadfence();
       if (atomicAdd(&a.counter[WS_DONE_WG], 1u) == gridDim.x - 1) {
         __threadfence();
-        if (atomicAdd(&a.counter[WS_DONE_ITEMS], 0u) != (unsigned)n_items) atomicOr(&a.counter[WS_STATUS], WS_SKIPPED);
+        if (atomicAdd(&a.counter[WS_DONE_ITEMS], 0u) != (unsigned)n_items ||
+            atomicAdd(&a.counter[WS_NEXT], 0u) != (unsigned)n_items)
+          atomicOr(&a.counter[WS_STATUS], WS_SKIPPED);
         atomicExch(&a.counter[WS_NEXT], 0u);
         atomicExch(&a.counter[WS_DONE_ITEMS], 0u);
         atomicExch(&a.counter[WS_DONE_WG], 0u);
@@ -1643,7 +1655,9 @@ static int prefill_impl(const char* fn, int dtype,
   a.row_order = (workspace != nullptr && csr_rows <= MAX_ORDERED_ROWS) ? 1 : 0;
   a.bhs = B * a.head_splits;
   a.q_split = 0;
-  if (a.row_order) {  // tail of about four items per persistent workgroup
+  // Tail of about four items per persistent workgroup.  Launches of at most LOOKAHEAD items per
+  // workgroup have no claims to balance: their items go out latest (heaviest) first throughout.
+  if (a.row_order && (int64_t)a.ntq * a.per_tile > LOOKAHEAD * (int64_t)num_cus()) {
     const int64_t tail = 4 * (int64_t)num_cus();
     a.q_split = (int)std::min<int64_t>(a.ntq, ceil_div(tail, a.per_tile));
   }
