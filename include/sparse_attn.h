@@ -89,7 +89,7 @@ const char* sa_last_error(void);
  * workspace is a status word that launches only set and the caller clears:
  * bit 0 means a launch's counters were not zero at launch or an overlapping
  * launch shared them: it may have processed fewer work items than it has and
- * left the skipped items' outputs unwritten.  NULL launches one workgroup per work
+ * left the skipped items' outputs unwritten; zero the whole workspace then.  NULL launches one workgroup per work
  * item instead.
  */
 int sa_prefill(int dtype,

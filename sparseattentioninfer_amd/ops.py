@@ -53,15 +53,16 @@ PREFILL_WS_SKIPPED = 1        # a launch processed fewer work items than it has
 
 def prefill_workspace_status(device=None, clear: bool = True) -> int:
     """Status word of the prefill workspace of the current stream on ``device`` (0: every launch
-    so far processed all its work items; bit 0: one did not, its output is incomplete).
-    Reads device memory (a synchronisation of the stream); ``clear`` resets the word."""
+    so far processed all its work items; bit 0: one may not have, its output is incomplete).
+    Reads device memory (a synchronisation of the stream); ``clear`` zeroes a workspace whose word
+    is set, counters included."""
     dev = torch.device("cuda", torch.cuda.current_device() if device is None else torch.device(device).index)
     ws = _PREFILL_WS.get((dev.index, torch.cuda.current_stream(dev).cuda_stream))
     if ws is None:
         return 0
     st = int(ws[PREFILL_WS_STATUS_WORD].item())
     if clear and st:
-        ws[PREFILL_WS_STATUS_WORD].zero_()
+        ws.zero_()
     return st
 
 
