@@ -20,13 +20,13 @@
 //  * four-head workgroups (8 waves, one per SIMD pair) run a software pipeline: the next
 //    tile's S^T = K Q^T is issued under the current tile's exponentials, and its row max
 //    under the current tile's O^T += V^T P^T; Q is staged in LDS there to leave the
-//    registers to the accumulators.  Smaller workgroups run one tile at a time;
+//    registers to the accumulators.  Smaller workgroups run one tile at a time, and split an
+//    item's tiles over slices of their waves where a launch has too few items for the chip;
 //  * the softmax works in base 2 with scale*log2(e) folded into one FMA before the
-//    hardware v_exp_f32 (2^x).  Four-head workgroups take each row's reference from its
-//    first tile's (masked) max and refit it (raise it to the tile max, rescale O and l)
-//    only when a lane's probabilities of one tile sum past 2^16 or overflow; smaller
-//    workgroups raise it when a row max exceeds it by more than 2^8.  Either way the
-//    common case never touches O with VALU;
+//    hardware v_exp_f32 (2^x).  A row's reference is the (masked) max of its first tile; it
+//    is refit (raised to the tile max, O and l rescaled) only when a lane's probabilities of
+//    one tile sum past 2^16 (2^15 in fp16) or overflow, so the common case never touches O
+//    with VALU;
 //  * the last tile of a four-head item skips the PV half (and the probabilities) of keys
 //    32..63 in a wave whose rows all end before them: the lower half on a diagonal tile;
 //  * O is written back through LDS so that every global store is a 16-byte piece of a
@@ -235,23 +235,10 @@ __device__ __forceinline__ void load_lds16(const void* vaddr, uint32_t lds) {
 // Waits for the calling wave's direct loads (and any other vector memory access).
 __device__ __forceinline__ void wait_dma() { __builtin_amdgcn_s_waitcnt(0x0F70); }  // vmcnt(0)
 
-// Wave-uniform 32-bit global read that has completed when it returns (it waits for every
-// vector memory access of the wave).  For the rare reads of a CSR row past its LDS cache:
-// written as one opaque block, it leaves the compiler no pending load into a register that
-// the LDS path reuses, which would otherwise make every LDS read of the row wait for the
-// direct loads.
-__device__ __forceinline__ int32_t load_uniform_now(const int32_t* p) {
-  int32_t x;
-  asm volatile(
-      "global_load_dword %0, %1, off\n\t"
-      "s_waitcnt vmcnt(0)"
-      : "=v"(x)
-      : "v"(p)
-      : "memory");
-  return __builtin_amdgcn_readfirstlane(x);
-}
-
-// Per-lane 32-bit global read that has completed when it returns (same reason as above).
+// Per-lane 32-bit global read that has completed when it returns (it waits for every vector memory
+// access of the wave).  For the rare reads of a CSR row past its LDS cache: written as one opaque
+// block, it leaves the compiler no pending load into a register that the LDS path reuses, which
+// would otherwise make every LDS read of the row wait for the direct loads.
 __device__ __forceinline__ int32_t load_lane_now(const int32_t* p) {
   int32_t x;
   asm volatile(
@@ -265,30 +252,34 @@ __device__ __forceinline__ int32_t load_lane_now(const int32_t* p) {
 
 // SUB: tile schedules with sub-block masks (block sizes 16 and 32); without it the mask
 // bookkeeping compiles away.  TL: the timeline instantiation (stamps compile away without it).
-template <bool BF16, int D, int HW, bool SUB, bool TL = false>
+template <bool BF16, int D, int HW, int NS, bool SUB, bool TL = false>
 struct Prefill {
   using E = Elem<BF16>;
-  static constexpr int NW = 2 * HW;              // waves: HW query heads x two 32-row halves
+  static constexpr int TW = 2 * HW;              // waves that share a K/V tile: HW query heads x two 32-row halves
+  static constexpr int NW = NS * TW;             // waves of the workgroup: NS slices
   static constexpr int NT = 64 * NW;             // threads
   static constexpr int NCG = D / 32;             // column groups of a staged tile
   static constexpr int TILE_BYTES = KT * D * 2;  // one staged K or V tile
   static constexpr int NI = TILE_BYTES / 1024;   // 1 KiB wave-wide direct loads per tile
-  static constexpr int NIW = NI / NW;            // ... issued by each wave
+  static constexpr int NIW = NI / TW;            // ... issued by each wave
   static constexpr int WAVE_BYTES = QT * D * 2;  // 32 rows of Q or O (one wave's share)
   // Four-head workgroups run the software-pipelined loop with K double- and V triple-
-  // buffered and Q staged in LDS.  Other shapes run one tile at a time over double-buffered
-  // K/V (single-buffered for one-head workgroups, so that more of them share a CU).
+  // buffered and Q staged in LDS.  Other shapes hold one K and one V tile per slice, each refilled
+  // as soon as it has been read (so four two-wave workgroups share a CU); slices merge their
+  // accumulators in fp32 through the same LDS.
   static constexpr bool PIPE = HW == 4;
-  static constexpr int NBK = PIPE ? 2 : (HW == 1 ? 1 : 2);
-  static constexpr int NBV = PIPE ? 3 : NBK;
-  static constexpr int LDS_KV = (NBK + NBV) * TILE_BYTES;
+  static constexpr int NBK = PIPE ? 2 : 1;
+  static constexpr int NBV = PIPE ? 3 : 1;
+  static constexpr int LDS_TILES = NS * (NBK + NBV) * TILE_BYTES;
+  static constexpr int LDS_MERGE = NS > 1 ? NW * QT * D * 4 : 0;
+  static constexpr int LDS_KV = LDS_TILES > LDS_MERGE ? LDS_TILES : LDS_MERGE;
   static constexpr int LDS_Q = PIPE ? NW * WAVE_BYTES : 16;
-  static constexpr float RESCALE_LOG2 = 8.f;
-  // Pipelined loop: the row reference is refit when one lane's probabilities of a tile (32 of a
-  // row's keys) sum past this; below it no probability exceeds 2^16, far from fp32 / bf16 overflow.
-  static constexpr float REFIT_SUM = 65536.f;
-  static_assert(NI % NW == 0, "direct loads must split evenly over the waves");
-  static_assert(NW * WAVE_BYTES <= LDS_KV, "the epilogue stages O in the K/V buffers");
+  // The row reference is refit when one lane's probabilities of a tile (32 of a row's keys) sum
+  // past this: no probability then exceeds 2^16 in bf16 (2^15 in fp16, whose largest is 65,504).
+  static constexpr float REFIT_SUM = BF16 ? 65536.f : 32768.f;
+  static_assert(NI % TW == 0, "direct loads must split evenly over the waves");
+  static_assert(NS == 1 || !PIPE, "four-head workgroups have one slice");
+  static_assert(TW * WAVE_BYTES <= (NBK + NBV) * TILE_BYTES, "the epilogue stages O in the K/V buffers");
   static_assert(!TL || PIPE, "the timeline instruments the persistent four-head loop");
 
   // TL only: charge the cycles since the last stamp to phase k (lane 0 of the first wave of each half).
@@ -449,10 +440,10 @@ struct Prefill {
     int q_row0, q_abs_tile_max, q_abs_min;
   };
 
-  // CSR entries of one row cached in LDS.  The persistent four-head loop keeps two rows
-  // (this item's and the next one's), so tile schedules, which also cache their masks, hold
-  // fewer entries per row there.
-  static constexpr int RC = (PIPE && SUB) ? ROW_CACHE / 2 : ROW_CACHE;
+  // CSR entries of one row cached in LDS.  The persistent loop keeps two rows (this item's and the
+  // next one's), so tile schedules, which also cache their masks, hold fewer entries per row, and
+  // so do the smaller workgroups, four of which share a CU's LDS.
+  static constexpr int RC = !PIPE ? ROW_CACHE / 4 : SUB ? ROW_CACHE / 2 : ROW_CACHE;
 
   // Work item (qt, r, hs, b) whose CSR row holds entries [e0, e0 + n_ent): pointers and
   // positions only, no memory reads.
@@ -461,7 +452,7 @@ struct Prefill {
     Item it;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = (tid >> 6) % TW;  // within the slice
     it.g = lane >> 5;
     it.l32 = lane & 31;
     const int hw = wave % HW;  // head within the workgroup
@@ -515,23 +506,13 @@ struct Prefill {
     return it.q_abs_tile_max < 0 ? -1 : min((a.Tk + KT - 1) / KT - 1, it.q_abs_tile_max / KT);
   }
 
-  // Key tile of schedule position t, or -1 for a negative block id or one past kt_hi's block
-  // (rejected before the shift, which cannot overflow then).
-  static __device__ __forceinline__ int tile_of(const PrefillArgs& a, const Item& it, const int32_t* s_row, int t,
-                                                int kt_hi) {
-    const int e = t >> a.tpb_log2;
-    // Two distinct loads (LDS cache, or a global read past the cached entries), so the two are
-    // not merged into one flat load of a selected pointer.
-    const int blk = it.cached ? s_row[e] : load_uniform_now(it.prow + it.e0 + e);
-    if (blk < 0 || blk > (kt_hi >> a.tpb_log2)) return -1;
-    return (blk << a.tpb_log2) + (t & it.tpb_mask);
-  }
-
   static __device__ __forceinline__ int sub_log2(const PrefillArgs& a) { return SUB ? a.sub_log2 : 0; }
 
-  // Sub-block mask of schedule position t (tile schedules only; t indexes entries there).
-  static __device__ __forceinline__ uint32_t mask_of(const Item& it, const int32_t* s_mask, int t) {
-    return (uint32_t)(it.cached ? s_mask[t] : load_uniform_now(it.mrow + it.e0 + t));
+  // Whether a sub-block mask keeps nothing for the 32 rows of half hf.
+  static __device__ __forceinline__ bool half_empty(const PrefillArgs& a, uint32_t m, int hf) {
+    if (!sub_log2(a)) return false;
+    const int n = (64 >> sub_log2(a)) * (QT >> sub_log2(a));  // bits of a half
+    return ((m >> (n * hf)) & ((1u << n) - 1u)) == 0;
   }
 
   // Whether a sub-block mask drops any sub-block of its tile.
@@ -556,23 +537,12 @@ struct Prefill {
     return ((bits >> sh) & 1u) ? lim : -1;
   }
 
-  // First tile at or after t that can contribute (0 <= kt <= kt_hi = kt_limit()): tiles entirely
-  // past T_k or above the causal limit of the whole 64-row query tile are skipped, and so are
-  // negative ids (malformed schedules) rather than read.
-  static __device__ __forceinline__ int next_usable(const PrefillArgs& a, const Item& it, const int32_t* s_row,
-                                                    int t, int kt_hi) {
-    for (; t < it.n_tiles; ++t) {
-      const int kt = tile_of(a, it, s_row, t, kt_hi);
-      if (kt >= 0 && kt <= kt_hi) break;
-    }
-    return t;
-  }
-
   // The usable tiles of an item in schedule order, read 64 schedule positions at a time:
   // lane i of `kt` holds the key tile of position `next - 64 + i` (and lane i of `m` its
   // sub-block mask), bit i of `live` marks it usable and not yet taken.  A tile is usable
-  // under the rule of next_usable: 0 <= kt <= kt_hi, the last key tile that starts before T_k
-  // and at or before the causal limit of the query tile.
+  // if 0 <= kt <= kt_hi, the last key tile that starts before T_k and at or before the causal
+  // limit of the query tile; negative ids and ids past it (malformed schedules) are skipped
+  // rather than read.
   struct TileQueue {
     int kt;
     uint32_t m;
@@ -703,154 +673,6 @@ struct Prefill {
     }
   }
 
-  // ---- one tile at a time (one- and two-head workgroups) -------------------------------
-  // Online softmax over the 32-key half j of the current tile for this wave's 32 rows.
-  // Scores are raw; p = 2^(s*c - m_ref).  Returns the P^T operands of the two 16-key chunks.
-  template <bool MASK>
-  static __device__ __forceinline__ void softmax_half(const PrefillArgs& a, f32x16& S, u32x4 (&P)[2],
-                                                      f32x16 (&O)[D / 32], float& m_ref, float& l_run, float c,
-                                                      uint32_t bits, int lim, int j) {
-    if (MASK) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int lh = chunk_lim(a, bits, lim, j, h);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int key = 32 * j + 16 * h + e;  // minus 8g, folded into the limit
-          if (key > lh) S[8 * h + e] = -__builtin_inff();
-        }
-      }
-    }
-    float mx = S[0];
-#pragma unroll
-    for (int rr = 1; rr < 16; ++rr) mx = fmaxf(mx, S[rr]);
-    mx = halves_max(mx);
-    const float m_tile = mx * c;  // -inf stays -inf (c > 0)
-    float m = m_ref == -__builtin_inff() ? m_tile : m_ref;
-    if (__any(m_tile > m + RESCALE_LOG2)) {
-      const float m_new = fmaxf(m, m_tile);
-      const float alpha = m_new == -__builtin_inff() ? 1.f : fast_exp2(m - m_new);
-      m = m_new;
-      l_run *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < D / 32; ++dt) O[dt] *= alpha;
-    }
-    m_ref = m;
-    const float neg_m = m == -__builtin_inff() ? 0.f : -m;
-    float ls = 0.f;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      float pf[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        pf[e] = fast_exp2(fmaf(S[8 * h + e], c, neg_m));
-        ls += pf[e];
-      }
-      P[h] = u32x4{E::pack2f(pf[0], pf[1]), E::pack2f(pf[2], pf[3]), E::pack2f(pf[4], pf[5]), E::pack2f(pf[6], pf[7])};
-    }
-    l_run += ls;
-  }
-
-  // One 64-key tile: S^T = K Q^T per 32-key half, softmax, O^T += V^T P^T.  The softmax of
-  // one half can run under the matrix instructions of the other half.
-  template <bool MASK>
-  static __device__ __forceinline__ void tile(const PrefillArgs& a, const char* cK, const char* cV, const Frag& f,
-                                              const u32x4 (&qf)[D / 16], f32x16 (&O)[D / 32], float& m_ref,
-                                              float& l_run, float c, uint32_t bits, int lim) {
-    // The two key halves are independent accumulation chains; alternating them keeps the
-    // matrix pipe busy while each MFMA waits for its predecessor's result.
-    f32x16 S[2] = {f32x16{}, f32x16{}};
-#pragma unroll
-    for (int cc = 0; cc < D / 16; ++cc)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) S[j] = E::mfma32(kfrag(cK, f, j, cc), qf[cc], S[j]);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      u32x4 P[2];
-      softmax_half<MASK>(a, S[j], P, O, m_ref, l_run, c, bits, lim, j);
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt) O[dt] = E::mfma32(vfrag(cV, f, j, h, dt), P[h], O[dt]);
-    }
-  }
-
-  // One work item, one tile at a time: the next tile's direct loads run under the current
-  // tile's compute (double buffer), or after it (single buffer).
-  static __device__ __forceinline__ void item(const PrefillArgs& a, int qt, int r, int hs, int b, char* sKV,
-                                              int32_t* s_row, int32_t* s_mask) {
-    char* sK = sKV;
-    char* sV = sKV + NBK * TILE_BYTES;
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const Item it = setup(a, qt, r, hs, b, s_row, s_mask);
-    // Q^T as the B operand of S^T = K Q^T: lane holds row l32, d = 16c + 8g .. +7.
-    u32x4 qf[D / 16];
-    {
-      const elem_t* qs = q_src(a, it);
-#pragma unroll
-      for (int c = 0; c < D / 16; ++c) qf[c] = *reinterpret_cast<const u32x4*>(qs + 16 * c);
-    }
-    const Frag f(lane);
-    const DmaLane dl(a, lane);
-    __syncthreads();  // s_row visible
-
-    f32x16 O[D / 32];
-#pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt) O[dt] = f32x16{};
-    float m_ref = -__builtin_inff();
-    float l_run = 0.f;  // this lane's half of the row sum
-    const float c = a.scale_log2;
-
-    const int kt_hi = kt_limit(a, it);
-    int t = next_usable(a, it, s_row, 0, kt_hi);
-    int buf = 0;
-    if (t < it.n_tiles) {
-      const int kt = tile_of(a, it, s_row, t, kt_hi);
-      dma<true>(it.kb, a.k_st, dl.k, sK, kt, a.Tk, wave, lane);
-      dma<false>(it.vb, a.v_st, dl.v, sV, kt, a.Tk, wave, lane);
-    }
-    wait_dma();
-    __syncthreads();
-
-    while (t < it.n_tiles) {
-      const int kt = tile_of(a, it, s_row, t, kt_hi);
-      const int tn = next_usable(a, it, s_row, t + 1, kt_hi);
-      if (NBK == 2 && tn < it.n_tiles) {
-        const int ktn = tile_of(a, it, s_row, tn, kt_hi);
-        dma<true>(it.kb, a.k_st, dl.k, sK + (buf ^ 1) * TILE_BYTES, ktn, a.Tk, wave, lane);
-        dma<false>(it.vb, a.v_st, dl.v, sV + (buf ^ 1) * TILE_BYTES, ktn, a.Tk, wave, lane);
-      }
-      const char* cK = sK + buf * TILE_BYTES;
-      const char* cV = sV + buf * TILE_BYTES;
-
-      // A wave whose 32 rows all precede the tile skips it (the other half may not).
-      if (kt * KT <= it.q_abs_min + QT - 1) {
-        const uint32_t m = sub_log2(a) ? mask_of(it, s_mask, t) : 0u;
-        const bool need_mask = (kt * KT + KT - 1 > it.q_abs_min) || (kt * KT + KT > a.Tk) || partial_mask(a, m);
-        const int lim = min(it.q_abs_min + it.l32, a.Tk - 1) - kt * KT - 8 * it.g;
-        const uint32_t bits = row_bits(a, m, it.hf, it.l32);
-        if (need_mask)
-          tile<true>(a, cK, cV, f, qf, O, m_ref, l_run, c, bits, lim);
-        else
-          tile<false>(a, cK, cV, f, qf, O, m_ref, l_run, c, bits, lim);
-      }
-
-      if (NBK == 1 && tn < it.n_tiles) {
-        __syncthreads();  // single buffer: every wave is done reading it
-        const int ktn = tile_of(a, it, s_row, tn, kt_hi);
-        dma<true>(it.kb, a.k_st, dl.k, sK, ktn, a.Tk, wave, lane);
-        dma<false>(it.vb, a.v_st, dl.v, sV, ktn, a.Tk, wave, lane);
-      }
-      wait_dma();
-      __syncthreads();
-      if (NBK == 2) buf ^= 1;
-      t = tn;
-    }
-    // Every wave has passed the last barrier: the K/V buffers are free for the staging.
-    epilogue(a, it, b, O, l_run, sKV + wave * WAVE_BYTES, lane);
-  }
-
   // ---- software-pipelined loop (four-head workgroups) ----------------------------------
   // Masks one tile's S^T (causal / past T_k / sub-blocks, branch-free): keys past the
   // chunk limits of (bits, lim) become -inf.
@@ -879,7 +701,7 @@ struct Prefill {
     return mx * c;  // -inf stays -inf (c > 0)
   }
 
-  // ---- lookahead metadata (persistent four-head loop) -----------------------------------
+  // ---- lookahead metadata (persistent loop) ---------------------------------------------
   // While an item's first tiles load, the persistent loop fetches the CSR row of the next
   // item, the CSR offsets and decoded (qt, r, hs, b) of the item after it and a new claim
   // from the counter.  All of it lands in LDS before the barrier that publishes the item's
@@ -955,6 +777,279 @@ struct Prefill {
       lk.meta2[6] = ld.b2;
       lk.vid3[0] = lk.taken ? claimed_item(a.claims, a.status, ld.nv, lk.taken, lk.fixed, lk.n_items) : lk.n_items;
     }
+  }
+
+  // ---- one- and two-head workgroups -----------------------------------------------------
+  // Writes this wave's accumulators (fp32), row references and row sums to LDS and merges the
+  // slices' shares of each row: slice s finishes columns s D / NS .. of every row of its wave pair.
+  // Accumulator row r is D fp32 at r * 4 D, its 16-byte chunk c at position c ^ (r % (D / 4)).
+  static __device__ __forceinline__ void epilogue_slices(const PrefillArgs& a, const Item& it, int b,
+                                                         const f32x16 (&O)[D / 32], float m_ref, float l_run, char* sKV,
+                                                         float* s_ml, int slice, int w2, int lane) {
+    constexpr int NC4 = D / 4;                  // fp32 chunks per row
+    constexpr int OC = D / 8 / NS;              // 16-byte output chunks per row and slice
+    constexpr int ACC_BYTES = QT * D * 4;       // one wave's accumulators
+    const int wave = slice * TW + w2;
+    char* acc = sKV + wave * ACC_BYTES;
+    const float lt = halves_sum(l_run);
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+      for (int rq = 0; rq < 4; ++rq) {  // d = 32dt + 8rq + 4g + 0..3: chunk 8dt + 2rq + g
+        const int c = 8 * dt + 2 * rq + it.g;
+        f32x4 w = {O[dt][4 * rq], O[dt][4 * rq + 1], O[dt][4 * rq + 2], O[dt][4 * rq + 3]};
+        *reinterpret_cast<f32x4*>(acc + it.l32 * 4 * D + 16 * (c ^ (it.l32 & (NC4 - 1)))) = w;
+      }
+    if (it.g == 0) {
+      s_ml[wave * 2 * QT + it.l32] = m_ref;
+      s_ml[wave * 2 * QT + QT + it.l32] = lt;
+    }
+    __syncthreads();
+    elem_t* ob = a.o + b * a.o_sb + it.hq * a.o_sh;
+#pragma unroll
+    for (int k = 0; k < QT * OC / 64; ++k) {
+      const int x = 64 * k + lane;
+      const int row = x / OC, oc = slice * OC + x % OC;
+      float m[NS], l = 0.f, M = -__builtin_inff();
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        m[s] = s_ml[(s * TW + w2) * 2 * QT + row];
+        M = fmaxf(M, m[s]);
+      }
+      const float Mu = M == -__builtin_inff() ? 0.f : M;
+      f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const float f = fast_exp2(m[s] - Mu);
+        l += f * s_ml[(s * TW + w2) * 2 * QT + QT + row];
+        const char* p = sKV + (s * TW + w2) * ACC_BYTES + row * 4 * D;
+        const f32x4 x0 = *reinterpret_cast<const f32x4*>(p + 16 * ((2 * oc) ^ (row & (NC4 - 1))));
+        const f32x4 x1 = *reinterpret_cast<const f32x4*>(p + 16 * ((2 * oc + 1) ^ (row & (NC4 - 1))));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          lo[e] += f * x0[e];
+          hi[e] += f * x1[e];
+        }
+      }
+      const float inv = l > 0.f ? 1.f / l : 1.f;
+      const u32x4 w = {E::pack2f(lo[0] * inv, lo[1] * inv), E::pack2f(lo[2] * inv, lo[3] * inv),
+                       E::pack2f(hi[0] * inv, hi[1] * inv), E::pack2f(hi[2] * inv, hi[3] * inv)};
+      if (it.q_row0 + row < a.Tq)
+        __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(ob + (int64_t)(it.q_row0 + row) * a.o_st + 8 * oc));
+    }
+  }
+
+  // One work item of a one- or two-head workgroup: per tile S^T = K Q^T, the probabilities, then
+  // O^T += V^T P^T.  The TW waves of a slice share one staged K and one staged V tile; slice s takes
+  // the item's usable tiles s, s + NS, ...  A wave whose 32 rows see nothing of a tile (causal limit,
+  // sub-block masks) only loads it: with blocks of 16 or 32 the two halves of a query tile keep mostly
+  // different blocks.
+  // With one slice four (two) workgroups share a CU and run at different points of their tiles, so a
+  // tile simply waits for its loads.  With slices the CU holds one workgroup (two with NS = 2), and its
+  // loads must run under its own work: K is refilled once every wave has read it (under the
+  // exponentials and the PV product), V after the PV product (under the next QK product).  That order
+  // costs two more barriers per tile and was slower with one slice: 8,192 tokens of 8 heads of 64,
+  // blocks of 16, 40.7 against 35.4 us.
+  // What bounds it (8,192 tokens, 32 heads of 128, blocks of 32): K/V tiles that feed one head, 3.4 GB
+  // staged of which 2.3 GB miss the L2s; 432 us before the lookahead, the skipped halves and the
+  // fourth workgroup per CU (smaller row caches), now 372 us.  A window of 512 keys, 4,096 tokens of
+  // 32 heads: 67 -> 59 us.
+  template <bool LOOK>
+  static __device__ __forceinline__ void item(const PrefillArgs& a, int qt, int r, int hs, int b, char* sKV,
+                                              float* s_ml, int32_t* s_row, int32_t* s_mask, const Look* lk) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int slice = NS == 1 ? 0 : wave / TW;
+    const int w2 = wave % TW;
+    char* sK = sKV + slice * 2 * TILE_BYTES;
+    char* sV = sK + TILE_BYTES;
+    const Item it = LOOK ? setup_base(a, qt, r, hs, b, lk->e0, lk->n_ent) : setup(a, qt, r, hs, b, s_row, s_mask);
+    // Q^T as the B operand of S^T = K Q^T: lane holds row l32, d = 16c + 8g .. +7.
+    u32x4 qf[D / 16];
+    {
+      const elem_t* qs = q_src(a, it);
+#pragma unroll
+      for (int c = 0; c < D / 16; ++c) qf[c] = *reinterpret_cast<const u32x4*>(qs + 16 * c);
+    }
+    const Frag f(lane);
+    const DmaLane dl(a, lane);
+    const int lim0 = min(it.q_abs_min + it.l32, a.Tk - 1) - 8 * it.g;
+    // The K/V buffers are free (every wave has finished the previous item) and s_row is visible.
+    __syncthreads();
+
+    f32x16 O[D / 32];
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt) O[dt] = f32x16{};
+    float m_ref = -__builtin_inff();
+    float neg_m = 0.f;
+    float l_run = 0.f;   // this lane's half of the row sum
+    bool ref_ok = false; // every row of the wave has a reference
+    const float c = a.scale_log2;
+
+    TileQueue q = queue_begin(a, it);
+    q.kt_hi = kt_limit(a, it);
+    // The next NS usable tiles, one per slice: whether there is any, and this slice's.
+    auto pop = [&](bool& has, int& kt, uint32_t& m) {
+      has = false;
+      bool any = false;
+#pragma unroll
+      for (int x = 0; x < NS; ++x) {
+        int k1 = 0;
+        uint32_t m1 = 0u;
+        const bool got = queue_pop(a, it, s_row, s_mask, q, k1, m1);
+        if (x == 0) any = got;
+        if (x == slice) {
+          has = got;
+          kt = k1;
+          m = m1;
+        }
+      }
+      return any;
+    };
+    auto load_k = [&](int kt) { dma<true>(it.kb, a.k_st, dl.k, sK, kt, a.Tk, w2, lane); };
+    auto load_v = [&](int kt) { dma<false>(it.vb, a.v_st, dl.v, sV, kt, a.Tk, w2, lane); };
+
+    bool has;
+    int kt = 0;
+    uint32_t m = 0u;
+    bool any = pop(has, kt, m);
+    if (has) {
+      load_k(kt);
+      load_v(kt);
+    }
+    // One wait for the first tiles and the lookahead's reads (and Q: with a load pending at the
+    // loop's entry the compiler would wait for every load in each step).
+    if constexpr (LOOK) {
+      LookLoads ld;
+      look_issue(a, *lk, ld);
+      wait_dma();
+      look_commit(a, *lk, ld);
+    } else {
+      wait_dma();
+    }
+    if (!any) __syncthreads();  // the lookahead's writes are visible (else by the first step's barrier)
+
+    // S^T = K Q^T of the tile: two independent accumulation chains keep the matrix pipe busy.
+    auto qk = [&](f32x16 (&S)[2]) {
+#pragma unroll
+      for (int cc = 0; cc < D / 16; ++cc)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) S[j] = E::mfma32(kfrag(sK, f, j, cc), qf[cc], S[j]);
+    };
+    // Raises each row's reference to its max over the keys of S (O and l rescaled to it).
+    auto refit = [&](const auto& S, auto nj_tag) {
+      constexpr int NJ = decltype(nj_tag)::value;
+      float mx = -__builtin_inff();
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int rr = 0; rr < 16; ++rr) mx = fmaxf(mx, S[j][rr]);
+      const float m_new = fmaxf(m_ref, halves_max(mx) * c);  // -inf stays -inf (c > 0)
+      const float alpha = m_ref == -__builtin_inff() ? 1.f : fast_exp2(m_ref - m_new);
+      l_run *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < D / 32; ++dt) O[dt] *= alpha;
+      m_ref = m_new;
+      neg_m = m_ref == -__builtin_inff() ? 0.f : -m_ref;
+      ref_ok = !__any(m_ref == -__builtin_inff());
+    };
+    // P^T operands of key half S against the row references; returns this lane's share of the sum.
+    auto probs = [&](const f32x16& S, u32x4 (&P)[2]) {
+      float ls = 0.f;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        uint32_t w[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float p0 = fast_exp2(fmaf(S[8 * h + 2 * e], c, neg_m));
+          const float p1 = fast_exp2(fmaf(S[8 * h + 2 * e + 1], c, neg_m));
+          ls += p0 + p1;
+          w[e] = E::pack2f(p0, p1);
+        }
+        P[h] = u32x4{w[0], w[1], w[2], w[3]};
+      }
+      return ls;
+    };
+    auto pv = [&](const u32x4 (&P)[2], int j) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int dt = 0; dt < D / 32; ++dt) O[dt] = E::mfma32(vfrag(sV, f, j, h, dt), P[h], O[dt]);
+    };
+
+    while (any) {
+      bool has_n;
+      int kt_n = 0;
+      uint32_t m_n = 0u;
+      const bool any_n = pop(has_n, kt_n, m_n);
+      const bool active = has && kt * KT <= it.q_abs_min + QT - 1 && !half_empty(a, m, it.hf);
+      const bool masked = kt * KT + KT - 1 > it.q_abs_min || kt * KT + KT > a.Tk || partial_mask(a, m);
+      f32x16 S[2] = {f32x16{}, f32x16{}};
+      u32x4 P[2][2];
+      // The probabilities are taken against the row reference; it is set by the first tile that shows
+      // the row a key and raised only when a lane's probabilities sum past REFIT_SUM or overflow.
+      if constexpr (NS == 1) {
+        wait_dma();
+        __syncthreads();  // K and V are in LDS
+        if (active) {
+          qk(S);
+          if (masked) mask_tile(a, S, row_bits(a, m, it.hf, it.l32), lim0 - kt * KT);
+          if (!ref_ok) refit(S, std::integral_constant<int, 2>{});
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            float ls = probs(S[j], P[j]);
+            if (__any(!(ls <= REFIT_SUM))) {
+              const f32x16 (&Sj)[1] = reinterpret_cast<const f32x16 (&)[1]>(S[j]);
+              refit(Sj, std::integral_constant<int, 1>{});
+              ls = probs(S[j], P[j]);
+            }
+            l_run += ls;
+            pv(P[j], j);
+          }
+        }
+        __syncthreads();  // both have been read
+        if (has_n) {
+          load_k(kt_n);
+          load_v(kt_n);
+        }
+      } else {
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (NIW & 15));  // vmcnt(NIW): K is in LDS, V may be in flight
+        __syncthreads();
+        if (active) qk(S);
+        __syncthreads();  // K has been read
+        if (has_n) load_k(kt_n);
+        if (active) {
+          if (masked) mask_tile(a, S, row_bits(a, m, it.hf, it.l32), lim0 - kt * KT);
+          if (!ref_ok) refit(S, std::integral_constant<int, 2>{});
+          float ls = probs(S[0], P[0]) + probs(S[1], P[1]);
+          if (__any(!(ls <= REFIT_SUM))) {
+            refit(S, std::integral_constant<int, 2>{});
+            ls = probs(S[0], P[0]) + probs(S[1], P[1]);
+          }
+          l_run += ls;
+        }
+        if (has_n)
+          __builtin_amdgcn_s_waitcnt(0x0F70 | (NIW & 15));  // V is in LDS, the next K may be in flight
+        else
+          wait_dma();
+        __syncthreads();
+        if (active) {
+          pv(P[0], 0);
+          pv(P[1], 1);
+        }
+        __syncthreads();  // V has been read
+        if (has_n) load_v(kt_n);
+      }
+      any = any_n;
+      has = has_n;
+      kt = kt_n;
+      m = m_n;
+    }
+    // Every wave has passed the last barrier: the K/V buffers are free for the staging.
+    if constexpr (NS == 1)
+      epilogue(a, it, b, O, l_run, sKV + wave * WAVE_BYTES, lane);
+    else
+      epilogue_slices(a, it, b, O, m_ref, l_run, sKV, s_ml, slice, w2, lane);
   }
 
   // Same work item as item(), with the tile loop software-pipelined: each step computes the
@@ -1341,7 +1436,7 @@ struct Prefill {
     b = __builtin_amdgcn_readfirstlane(b);
   }
 
-  static __device__ __forceinline__ void process(const PrefillArgs& a, int v, char* sKV, char* sQ,
+  static __device__ __forceinline__ void process(const PrefillArgs& a, int v, char* sKV, char* sQ, float* s_ml,
                                                  int32_t* s_row, int32_t* s_mask) {
     int qt, r, hs, b;
     decode_item_uniform(a, v, qt, r, hs, b);
@@ -1351,10 +1446,10 @@ struct Prefill {
       item_pipelined<false>(a, qt, r, hs, b, sKV, sQ, s_row, s_mask, nullptr, vb_first);
     }
     else
-      item(a, qt, r, hs, b, sKV, s_row, s_mask);
+      item<false>(a, qt, r, hs, b, sKV, s_ml, s_row, s_mask, nullptr);
   }
 
-  // Persistent four-head loop with lookahead.  The first LOOKAHEAD items of a workgroup w are fixed
+  // Persistent loop with lookahead.  The first LOOKAHEAD items of a workgroup w are fixed
   // by w, later ones are claimed from the counter.  (Claimed ahead, the first ones all went to the
   // workgroups that started first, three each: 128 items of 64-79 tiles -- 1,000 queries of 32
   // heads on 5,000 keys -- ran on 43 CUs, 297 us; one item per workgroup takes 107 us.)  With fewer
@@ -1369,7 +1464,7 @@ struct Prefill {
   // (Look).  Claims only grow, so the first id past the end ends the loop in every wave at
   // once.
   static __device__ __forceinline__ void run_lookahead(const PrefillArgs& a, int n_items, char* sKV, char* sQ,
-                                                      int32_t* s_row, int32_t* s_mask) {
+                                                       float* s_ml, int32_t* s_row, int32_t* s_mask) {
     int vb_first = 0;  // V buffer free for the next item's first tile
     // Per slot k = item index mod 4: id, CSR offsets (first, end) and (qt, r, hs, b); the loop
     // top reads an item's whole slot (and the ids and offsets of the next two) in one batch.
@@ -1444,19 +1539,22 @@ struct Prefill {
       const int r = __builtin_amdgcn_readfirstlane(m0b.x);
       const int hs = __builtin_amdgcn_readfirstlane(m0b.y);
       const int b = __builtin_amdgcn_readfirstlane(m0b.z);
-      item_pipelined<true>(a, qt, r, hs, b, sKV, sQ, s_row + (i & 1) * RC, SUB ? s_mask + (i & 1) * RC : s_mask,
-                           &lk, vb_first);
+      int32_t* row = s_row + (i & 1) * RC;
+      int32_t* mask = SUB ? s_mask + (i & 1) * RC : s_mask;
+      if constexpr (PIPE)
+        item_pipelined<true>(a, qt, r, hs, b, sKV, sQ, row, mask, &lk, vb_first);
+      else
+        item<true>(a, qt, r, hs, b, sKV, s_ml, row, mask, &lk);
     }
   }
 
   static __device__ void run(const PrefillArgs& a) {
     __shared__ __attribute__((aligned(16))) char sKV[LDS_KV];
     __shared__ __attribute__((aligned(16))) char sQ[LDS_Q];
-    // Row caches: two for the persistent four-head loop (this item and the next one).
-    constexpr int NROW = PIPE ? 2 : 1;
-    __shared__ int32_t s_row[NROW * RC];
-    __shared__ int32_t s_mask[SUB ? NROW * RC : 1];  // sub-block masks of the cached rows
-    __shared__ int s_item;
+    __shared__ float s_ml[NS > 1 ? NW * 2 * QT : 1];  // the slices' row references and sums
+    // Row caches: two for the persistent loop (this item and the next one).
+    __shared__ int32_t s_row[2 * RC];
+    __shared__ int32_t s_mask[SUB ? 2 * RC : 1];  // sub-block masks of the cached rows
     const int n_items = a.ntq * a.R * a.B * a.head_splits;
 
     if (!a.claims) {
@@ -1469,7 +1567,7 @@ struct Prefill {
       const int xcd = blockIdx.x % N_XCD, seq = blockIdx.x / N_XCD;
       const int v = ((seq / chunk) * N_XCD + xcd) * chunk + seq % chunk;
       if (v >= n_items) return;  // padding workgroup of the last round
-      process(a, v, sKV, sQ, s_row, s_mask);
+      process(a, v, sKV, sQ, s_ml, s_row, s_mask);
       return;
     }
 
@@ -1487,32 +1585,20 @@ struct Prefill {
       if (wave % HW == 0 && (threadIdx.x & 63) == 0) s_tl[wave / HW][TL_NOW] = (unsigned)__builtin_amdgcn_s_memtime();
     }
     if (a.row_order) rank_rows(a, reinterpret_cast<int*>(sKV));  // K/V buffers are free here
-    const int fixed = (PIPE ? LOOKAHEAD : 1) * (int)gridDim.x;
+    const int fixed = LOOKAHEAD * (int)gridDim.x;
     // All items dealt: no workgroup claims, and one looks whether the claims word was zero (read
     // here, looked at after its items, so nothing waits for it).
     unsigned long long seen = 0;
     if (n_items <= fixed && blockIdx.x == 0 && threadIdx.x == 0)
       seen = __hip_atomic_load(a.claims, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if constexpr (PIPE) {
-      run_lookahead(a, n_items, sKV, sQ, s_row, s_mask);
-      if constexpr (TL) {
-        __syncthreads();  // every stamp is in LDS
-        if (threadIdx.x == 0) {
-          rec[2] = __builtin_amdgcn_s_memtime();
-          rec[3] = __builtin_amdgcn_s_memrealtime();
-        }
-        if (threadIdx.x < 2 * TL_HALF_WORDS) rec[4 + threadIdx.x] = s_tl[threadIdx.x / TL_HALF_WORDS][threadIdx.x % TL_HALF_WORDS];
+    run_lookahead(a, n_items, sKV, sQ, s_ml, s_row, s_mask);
+    if constexpr (TL) {
+      __syncthreads();  // every stamp is in LDS
+      if (threadIdx.x == 0) {
+        rec[2] = __builtin_amdgcn_s_memtime();
+        rec[3] = __builtin_amdgcn_s_memrealtime();
       }
-    } else {
-      __syncthreads();  // row ranks visible, and the K/V buffers they were computed in free
-      for (int v = (int)blockIdx.x; v < n_items;) {  // the first item is this workgroup's own
-        process(a, v, sKV, sQ, s_row, s_mask);
-        if (n_items <= fixed) break;
-        if (threadIdx.x == 0) s_item = claimed_item(a.claims, a.status, add_claim(a.claims, 1), 1, fixed, n_items);
-        __syncthreads();
-        v = s_item;
-        __syncthreads();
-      }
+      if (threadIdx.x < 2 * TL_HALF_WORDS) rec[4 + threadIdx.x] = s_tl[threadIdx.x / TL_HALF_WORDS][threadIdx.x % TL_HALF_WORDS];
     }
     if (seen != 0) {
       atomicExch(a.claims, 0ull);
@@ -1522,28 +1608,28 @@ struct Prefill {
 };
 
 // At most 256 registers per wave: two waves per SIMD (one 8-wave workgroup per CU).
-template <bool BF16, int D, int HW, bool SUB>
-__global__ __launch_bounds__(128 * HW) __attribute__((amdgpu_waves_per_eu(2)))
+template <bool BF16, int D, int HW, int NS, bool SUB>
+__global__ __launch_bounds__(128 * HW * NS) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_kernel(PrefillArgs a) {
-  Prefill<BF16, D, HW, SUB>::run(a);
+  Prefill<BF16, D, HW, NS, SUB>::run(a);
 }
 
 // The timeline instantiation of the persistent four-head kernel (head dim 128, blocks of 64 or 128).
 template <bool BF16>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_timeline_kernel(PrefillArgs a) {
-  Prefill<BF16, 128, 4, false, true>::run(a);
+  Prefill<BF16, 128, 4, 1, false, true>::run(a);
 }
 
 // Resident workgroups of one kernel instance per CU, and CUs, cached per device.
-template <bool BF16, int D, int HW, bool SUB>
+template <bool BF16, int D, int HW, int NS, bool SUB>
 static int resident_per_cu() {
   static int cached[64] = {0};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 1;
   if (!cached[dev]) {
     int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, prefill_kernel<BF16, D, HW, SUB>, 128 * HW, 0) != hipSuccess || n < 1)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, prefill_kernel<BF16, D, HW, NS, SUB>, 128 * HW * NS, 0) != hipSuccess || n < 1)
       n = 1;
     cached[dev] = n;
   }
@@ -1562,26 +1648,29 @@ static int num_cus() {
   return cached[dev];
 }
 
-template <bool BF16, int D, int HW, bool SUB>
+template <bool BF16, int D, int HW, int NS, bool SUB>
 static hipError_t launch_sub(const PrefillArgs& a, int64_t n_items, int64_t item_grid, hipStream_t s) {
   int64_t grid = item_grid;
-  if (a.claims) grid = std::min<int64_t>(n_items, (int64_t)num_cus() * resident_per_cu<BF16, D, HW, SUB>());
-  hipLaunchKernelGGL((prefill_kernel<BF16, D, HW, SUB>), dim3(grid), dim3(128 * HW), 0, s, a);
+  if (a.claims) grid = std::min<int64_t>(n_items, (int64_t)num_cus() * resident_per_cu<BF16, D, HW, NS, SUB>());
+  hipLaunchKernelGGL((prefill_kernel<BF16, D, HW, NS, SUB>), dim3(grid), dim3(128 * HW * NS), 0, s, a);
   return hipGetLastError();
 }
 
-template <bool BF16, int D, int HW>
+template <bool BF16, int D, int HW, int NS>
 static hipError_t launch_hw(const PrefillArgs& a, int64_t n_items, int64_t item_grid, hipStream_t s) {
-  return a.sub_log2 ? launch_sub<BF16, D, HW, true>(a, n_items, item_grid, s)
-                    : launch_sub<BF16, D, HW, false>(a, n_items, item_grid, s);
+  return a.sub_log2 ? launch_sub<BF16, D, HW, NS, true>(a, n_items, item_grid, s)
+                    : launch_sub<BF16, D, HW, NS, false>(a, n_items, item_grid, s);
 }
 
 template <bool BF16, int D>
-static hipError_t launch_d(const PrefillArgs& a, int hw, int64_t n_items, int64_t item_grid, hipStream_t s) {
-  switch (hw) {
-    case 4: return launch_hw<BF16, D, 4>(a, n_items, item_grid, s);
-    case 2: return launch_hw<BF16, D, 2>(a, n_items, item_grid, s);
-    default: return launch_hw<BF16, D, 1>(a, n_items, item_grid, s);
+static hipError_t launch_d(const PrefillArgs& a, int hw, int ns, int64_t n_items, int64_t item_grid, hipStream_t s) {
+  switch (10 * hw + ns) {
+    case 41: return launch_hw<BF16, D, 4, 1>(a, n_items, item_grid, s);
+    case 22: return launch_hw<BF16, D, 2, 2>(a, n_items, item_grid, s);
+    case 21: return launch_hw<BF16, D, 2, 1>(a, n_items, item_grid, s);
+    case 14: return launch_hw<BF16, D, 1, 4>(a, n_items, item_grid, s);
+    case 12: return launch_hw<BF16, D, 1, 2>(a, n_items, item_grid, s);
+    default: return launch_hw<BF16, D, 1, 1>(a, n_items, item_grid, s);
   }
 }
 
@@ -1594,6 +1683,34 @@ static int64_t timeline_grid(bool bf16) {
                             : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, prefill_timeline_kernel<false>, 512, 0);
   if (e != hipSuccess || n < 1) n = 1;
   return (int64_t)num_cus() * n;
+}
+
+// Heads per workgroup and slices of its waves.  Heads that share a CSR row share its K/V tiles, four
+// of them in the pipelined kernel, as long as the launch fills the chip (`waves`: two per head, CSR
+// row and query tile; a CU runs eight).  Launches that leave CUs or their SIMDs idle give an item's
+// tiles to several slices of one workgroup instead.  Measured (us; heads per row, tile lists):
+//   items of one head, 8 heads of 64, BigBird blocks of 16 (<= 19 tiles): 128 items 23.5 / 19.4 / 16.1
+//   with 1 / 2 / 4 slices, 504 items 31.8 / 27.6 / 35.1, 1,000 items 35.4 / 52.4 / 70.5; head dim 128,
+//   256 items of 9 tiles 21.3 / 17.5 / 17.1, 512 items 25.8 / 23.3 / 32.2, 1,024 items 37.1 / 42.1 / 63.3;
+//   two heads, 1,000 queries on 5,000 keys: 136.5 with (2, 1), 101.3 with (2, 2), 68.5 with (1, 4)
+//   (512 waves); 2,048 queries 178.7 / 126.8 / 138.3 (1,024 waves), 4,096 queries 265.7 / 263.5 / 427.7;
+//   four heads, 512 queries on 4,512 keys (512 waves): 97.9 pipelined, 62.7 with (1, 4); 1,000 queries
+//   114.7 / 127.7; BigBird of 8 tiles, 512 tokens (512 waves) 17.5 / 13.4, 1,000 tokens 18.8 / 23.9.
+// Four-head launches with at most 15 key tiles stay pipelined: there is little to divide.
+struct Shape {
+  int hw, ns;
+};
+
+static Shape choose_shape(int T_q, int T_k, int rows, int B, int heads_per_row) {
+  const int64_t waves = 2 * ceil_div(T_q, QTILE) * rows * (int64_t)B * heads_per_row;
+  const int64_t cus = num_cus();
+  if (heads_per_row % 4 == 0) {
+    if (waves <= 2 * cus && T_k > 15 * KT) return {1, 4};
+    return {4, 1};
+  }
+  if (waves <= 2 * cus) return {1, 4};
+  const int hw = heads_per_row % 2 == 0 ? 2 : 1;
+  return {hw, waves <= 4 * cus ? 2 : 1};
 }
 
 static int prefill_impl(const char* fn, int dtype,
@@ -1659,7 +1776,9 @@ static int prefill_impl(const char* fn, int dtype,
   a.sub_log2 = block_size == 16 ? 4 : block_size == 32 ? 5 : 0;
   a.R = csr_rows;
   a.heads_per_row = Hq / csr_rows;
-  const int hw = (a.heads_per_row % 4 == 0) ? 4 : (a.heads_per_row % 2 == 0) ? 2 : 1;
+  const Shape shape = timeline ? Shape{(a.heads_per_row % 4 == 0) ? 4 : 1, 1}
+                               : choose_shape(T_q, T_k, csr_rows, B, a.heads_per_row);
+  const int hw = shape.hw, ns = shape.ns;
   a.head_splits = a.heads_per_row / hw;
   a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.Tq = T_q; a.Tk = T_k;
   a.ntq = (int)ceil_div(T_q, QTILE);
@@ -1674,8 +1793,9 @@ static int prefill_impl(const char* fn, int dtype,
   a.q_split = 0;
   // Tail of about four items per persistent workgroup.  Launches of at most LOOKAHEAD items per
   // workgroup have no claims to balance: their items go out latest (heaviest) first throughout.
-  if (a.row_order && (int64_t)a.ntq * a.per_tile > LOOKAHEAD * (int64_t)num_cus()) {
-    const int64_t tail = 4 * (int64_t)num_cus();
+  const int64_t resident = (int64_t)num_cus() * std::max(1, 4 / (hw * ns));  // workgroups, about
+  if (a.row_order && (int64_t)a.ntq * a.per_tile > LOOKAHEAD * resident) {
+    const int64_t tail = 4 * resident;
     a.q_split = (int)std::min<int64_t>(a.ntq, ceil_div(tail, a.per_tile));
   }
   if (a.q_split == 0) a.row_order = 0;
@@ -1722,9 +1842,9 @@ static int prefill_impl(const char* fn, int dtype,
       hipLaunchKernelGGL((prefill_timeline_kernel<false>), dim3(grid), dim3(512), 0, s, a);
     err = hipGetLastError();
   } else if (D == 128)
-    err = bf16 ? launch_d<true, 128>(a, hw, n_items, item_grid, s) : launch_d<false, 128>(a, hw, n_items, item_grid, s);
+    err = bf16 ? launch_d<true, 128>(a, hw, ns, n_items, item_grid, s) : launch_d<false, 128>(a, hw, ns, n_items, item_grid, s);
   else
-    err = bf16 ? launch_d<true, 64>(a, hw, n_items, item_grid, s) : launch_d<false, 64>(a, hw, n_items, item_grid, s);
+    err = bf16 ? launch_d<true, 64>(a, hw, ns, n_items, item_grid, s) : launch_d<false, 64>(a, hw, ns, n_items, item_grid, s);
   if (err != hipSuccess) return set_error((int)err, "%s: launch failed: %s", fn, hipGetErrorString(err));
   return 0;
 }
