@@ -275,6 +275,13 @@ def universal_sparse_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     lib = _lib.load()
     if T_q == 1 and q_offset == T_k - 1:
         _require(nqb == 1, f"{name}: decode expects one CSR query block, got {nqb}")
+        # Lists of 1,024 keys and more are split over workgroups: unsplit, a row's list is read by one CU
+        # (4 sequences of 8,191 tokens, 32 heads, 8 KV heads: 137 us; split by 8, 27 us).  Shorter ones are
+        # not: the partials and the combine cost an eager call 5 us of launching (256 keys of 8 heads: 15 us
+        # unsplit, 20 us split by 8).
+        splits = _decode_splits(_decode_units(B, Hq, R), pairs.size(1)) if pairs.size(1) * block_size >= 1024 else 1
+        ws_bytes = splits * B * Hq * (D + 2) * 4 if splits > 1 else 0
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
         status = lib.sa_decode(
             _DTYPES[q.dtype],
             q.data_ptr(), q.stride(0), q.stride(1),
@@ -286,7 +293,7 @@ def universal_sparse_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
             R,
             out.data_ptr(), out.stride(0), out.stride(1),
             B, Hq, Hkv, D, block_size, sm_scale,
-            1, None, 0, _stream(q))
+            splits, ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q))
         _lib.check("sa_decode", status)
         return out
     _require(block_size <= 128, f"{name}: block_size {block_size} not supported by the "
@@ -339,6 +346,25 @@ def auto_decode_splits(B: int, rows: int, max_sel: int, target_workgroups: int =
     return max(1, min(want, max_sel // 2, 16))
 
 
+def _decode_splits(units: int, max_sel: int) -> int:
+    """Splits of each block list for one decode launch of ``units`` workgroups unsplit: up to one
+    workgroup per CU (256), at least two blocks per split, at most 32 splits.
+
+    A workgroup's four waves keep about 64 KB of loads in flight, so 256 of them already draw HBM's
+    rate and further splits only add to the combine.  Measured (us): 4 sequences of 8,191 tokens (32
+    units, 134 MB) 41.7 / 27.1 / 28.5 / 34.2 with 4 / 8 / 16 / 32 splits; one of 32,000 (8 units) 72.9 /
+    42.0 / 28.8 / 31.9 with 8 / 16 / 32 / 64; 14 blocks of 64 kept by 64 units 19.5 / 15.3 / 13.3 / 13.2
+    with 1 / 2 / 4 / 8, by 128 units 20.1 / 17.6 / 19.0 with 1 / 2 / 4, by 192 units 22.0 / 25.2 with 1 / 2.
+    """
+    return max(1, min(256 // max(1, units), max_sel // 2, 32))
+
+
+def _decode_units(B: int, Hq: int, rows: int) -> int:
+    """Workgroups of an unsplit decode launch: up to four query heads of a row share one."""
+    per_row = Hq // rows
+    return B * rows * (per_row // 4 if per_row % 4 == 0 else per_row // 2 if per_row % 2 == 0 else per_row)
+
+
 def paged_sparse_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
                         block_table: torch.Tensor, kv_lens: torch.Tensor,
                         sel: torch.Tensor, sel_off: torch.Tensor, *,
@@ -352,7 +378,7 @@ def paged_sparse_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.T
     [B, R, 2]`` int32 retained logical blocks per (sequence, row), R = Hq or
     Hkv.  ``num_splits > 1`` splits each row over workgroups and needs a
     byte workspace of :func:`decode_workspace_bytes` (allocated if omitted);
-    ``num_splits=0`` picks the count with :func:`auto_decode_splits`.
+    ``num_splits=0`` picks the count from the shapes.
     """
     name = "paged_sparse_decode"
     q3 = q.reshape(q.shape[0], q.shape[1], q.shape[-1]) if q.dim() == 4 else q
@@ -374,7 +400,7 @@ def paged_sparse_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.T
     _require(sel.stride(2) == 1 and block_table.stride(1) == 1 and kv_lens.is_contiguous()
              and sel_off.stride(2) == 1, f"{name}: index tensors must be contiguous in the last dim")
     if num_splits == 0:
-        num_splits = auto_decode_splits(B, R, sel.shape[2])
+        num_splits = _decode_splits(_decode_units(B, Hq, R), sel.shape[2])
     if out is None:
         out = torch.empty(B, Hq, D, dtype=q3.dtype, device=q3.device)
     lib = _lib.load()

@@ -1,0 +1,44 @@
+"""Contiguous decode (``universal_sparse_attn`` with one query) around the list lengths from which a
+block list is split over workgroups: just below and at 1,024 keys, lists of a few blocks more than the
+splits, the 32-split cap, ragged last blocks; and the paged entry point's own choice (``num_splits=0``)."""
+import sys
+
+import pytest
+import torch
+
+from oracle import attention as oa
+from sparseattentioninfer_amd import ops
+from sparseattentioninfer_amd.patterns import block_mask_to_csr
+from tests.helpers import assert_close_bf16, seeded
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,rows,D,bs,T", [
+    (1, 8, 2, 2, 128, 64, 959), (1, 8, 2, 2, 128, 64, 961), (1, 8, 2, 8, 128, 64, 1025), (2, 6, 3, 3, 64, 16, 1024),
+    (1, 4, 1, 1, 128, 64, 4480), (1, 4, 1, 1, 64, 128, 9000), (3, 16, 2, 2, 128, 32, 2051), (40, 8, 8, 8, 64, 64, 1500)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_split_decode_matches_the_oracle(B, Hq, Hkv, rows, D, bs, T, dtype):
+    print(f"[decode splits] B={B} heads={Hq}/{Hkv} rows={rows} D={D} bs={bs} T={T} {dtype}", flush=True)
+    sys.stdout.flush()
+    nkb = -(-T // bs)
+    bm = torch.ones(rows, 1, nkb, dtype=torch.bool)
+    bm[0, 0, 1::3] = False                                 # rows of different lengths
+    pairs, offsets = block_mask_to_csr(bm)
+    q = seeded((B, Hq, 1, D), 1, dtype).to(DEV)
+    k, v = (seeded((B, Hkv, T + 70, D), s, dtype).to(DEV)[:, :, :T] for s in (2, 3))   # a cache's views
+    out = ops.universal_sparse_attn(q, k, v, pairs.to(DEV), offsets.to(DEV), bs)
+    want = oa.block_sparse_attention(q, k, v, pairs, offsets, bs)
+    assert_close_bf16(out, want, "contiguous")
+    if T % bs == 0 or bs > 64 or B > 3:
+        return
+    # the same lists over pages, split count chosen from the shapes
+    pad = torch.zeros(B, Hkv, nkb * bs - T, D, dtype=dtype, device=DEV)
+    kp, vp = (torch.cat([x, pad], 2).reshape(B, Hkv, nkb, bs, D).transpose(1, 2).reshape(B * nkb, Hkv, bs, D).contiguous()
+              for x in (k, v))
+    table = torch.arange(B * nkb, dtype=torch.int32, device=DEV).reshape(B, nkb)
+    got = ops.paged_sparse_decode(q, kp, vp, table, torch.full((B,), T, dtype=torch.int32, device=DEV),
+                                  pairs.to(DEV)[None].expand(B, -1, -1), offsets.to(DEV)[None].expand(B, -1, -1),
+                                  num_splits=0)
+    assert_close_bf16(got, want, "paged")
