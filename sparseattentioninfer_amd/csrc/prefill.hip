@@ -1791,11 +1791,14 @@ static int prefill_impl(const char* fn, int dtype,
   a.row_order = (workspace != nullptr && csr_rows <= MAX_ORDERED_ROWS) ? 1 : 0;
   a.bhs = B * a.head_splits;
   a.q_split = 0;
-  // Tail of about four items per persistent workgroup.  Launches of at most LOOKAHEAD items per
+  // Tail of about four items per four-head workgroup, and of half an item per smaller one: with a
+  // schedule per head, all heads of a query tile in flight together find more of their K/V in the
+  // L2s than whole rows after one another do (8,192 tokens, 32 heads, blocks of 32: 339 us, with
+  // two or four items per workgroup 375; 3 x 2,730 tokens 249 against 273 and 320 us).  Launches of at most LOOKAHEAD items per
   // workgroup have no claims to balance: their items go out latest (heaviest) first throughout.
   const int64_t resident = (int64_t)num_cus() * std::max(1, 4 / (hw * ns));  // workgroups, about
   if (a.row_order && (int64_t)a.ntq * a.per_tile > LOOKAHEAD * resident) {
-    const int64_t tail = 4 * resident;
+    const int64_t tail = hw == 4 ? 4 * resident : resident / 2;
     a.q_split = (int)std::min<int64_t>(a.ntq, ceil_div(tail, a.per_tile));
   }
   if (a.q_split == 0) a.row_order = 0;
