@@ -106,6 +106,35 @@ int sa_prefill(int dtype,
                void* workspace, int64_t workspace_bytes,
                void* stream);
 
+/*
+ * sa_prefill with an optional buffer for partial results (16-byte aligned,
+ * contents arbitrary): with sa_prefill_partial_bytes() bytes of it (and a
+ * workspace), launches whose query tiles are few and whose block lists are
+ * long divide each query tile's keys over several workgroups and merge their
+ * fp32 partials with a second kernel.  Without it, or where that function
+ * returns 0, it is sa_prefill.  Calls that may run concurrently need a buffer
+ * each.
+ */
+int sa_prefill_split(int dtype,
+                     const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st,
+                     const void* k, int64_t k_sb, int64_t k_sh, int64_t k_st,
+                     const void* v, int64_t v_sb, int64_t v_sh, int64_t v_st,
+                     void* o, int64_t o_sb, int64_t o_sh, int64_t o_st,
+                     const int32_t* pairs, int64_t pairs_stride,
+                     const int32_t* offsets, int64_t offsets_stride,
+                     const int32_t* tile_masks, int64_t tile_masks_stride,
+                     int csr_rows, int nqb,
+                     int B, int Hq, int Hkv, int T_q, int T_k, int D,
+                     int block_size, int q_offset, float sm_scale,
+                     void* workspace, int64_t workspace_bytes,
+                     void* partials, int64_t partials_bytes,
+                     void* stream);
+
+/* Bytes of partials that a sa_prefill_split call of these sizes uses (0: none);
+ * pairs_stride as passed to the call. */
+int64_t sa_prefill_partial_bytes(int csr_rows, int B, int Hq, int T_q, int T_k, int D, int block_size,
+                                 int64_t pairs_stride);
+
 /* Bytes of the optional sa_prefill workspace (counters and the status word). */
 int64_t sa_prefill_workspace_bytes(void);
 

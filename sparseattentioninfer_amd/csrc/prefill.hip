@@ -31,6 +31,8 @@
 //    32..63 in a wave whose rows all end before them: the lower half on a diagonal tile;
 //  * O is written back through LDS so that every global store is a 16-byte piece of a
 //    contiguous row;
+//  * four-head launches of few query tiles with long lists divide each item's keys over
+//    workgroups, whose fp32 partials a second kernel merges;
 //  * with a workspace, one persistent workgroup per CU slot takes its first work items by its
 //    own index and claims further ones from an atomic counter, heaviest query tiles first.
 //
@@ -105,6 +107,12 @@ struct PrefillArgs {
   int nqb;
   int q_split, head_items, per_group, bhs;
   uint32_t mul_group, mul_bhs;
+  // Key splits (KS): work item v is split v % splits of item v / splits; it takes the item's usable
+  // tiles within its share of the key tiles before the item's limit, and leaves fp32 partials
+  // (part_words per wave) that prefill_combine_kernel merges.
+  int splits;
+  uint32_t mul_splits;
+  float* part;
   // Timeline launches only (sa_prefill_timeline): TL_WORDS words per workgroup.
   unsigned long long* timeline;
 };
@@ -252,7 +260,8 @@ __device__ __forceinline__ int32_t load_lane_now(const int32_t* p) {
 
 // SUB: tile schedules with sub-block masks (block sizes 16 and 32); without it the mask
 // bookkeeping compiles away.  TL: the timeline instantiation (stamps compile away without it).
-template <bool BF16, int D, int HW, int NS, bool SUB, bool TL = false>
+// KS: key splits (see PrefillArgs::splits; four-head workgroups).
+template <bool BF16, int D, int HW, int NS, bool SUB, bool TL = false, bool KS = false>
 struct Prefill {
   using E = Elem<BF16>;
   static constexpr int TW = 2 * HW;              // waves that share a K/V tile: HW query heads x two 32-row halves
@@ -280,6 +289,7 @@ struct Prefill {
   static_assert(NI % TW == 0, "direct loads must split evenly over the waves");
   static_assert(NS == 1 || !PIPE, "four-head workgroups have one slice");
   static_assert(TW * WAVE_BYTES <= (NBK + NBV) * TILE_BYTES, "the epilogue stages O in the K/V buffers");
+  static_assert(!KS || PIPE, "key splits are for four-head workgroups");
   static_assert(!TL || PIPE, "the timeline instruments the persistent four-head loop");
 
   // TL only: charge the cycles since the last stamp to phase k (lane 0 of the first wave of each half).
@@ -549,6 +559,7 @@ struct Prefill {
     uint64_t live;
     int next;
     int kt_hi;
+    int kt_lo;  // KS only
   };
 
   static __device__ __forceinline__ TileQueue queue_begin(const PrefillArgs& a, const Item& it) {
@@ -575,7 +586,7 @@ struct Prefill {
     const bool ok = blk >= 0 && blk <= (q.kt_hi >> a.tpb_log2);
     q.kt = ok ? blk * (1 << a.tpb_log2) + (t & it.tpb_mask) : -1;
     q.m = m;
-    q.live = __builtin_amdgcn_ballot_w64(ok && q.kt <= q.kt_hi);
+    q.live = __builtin_amdgcn_ballot_w64(ok && q.kt <= q.kt_hi && (!KS || q.kt >= q.kt_lo));
     q.next += 64;
   }
 
@@ -670,6 +681,91 @@ struct Prefill {
         const u32x4 w = *reinterpret_cast<const u32x4*>(stage + row * 2 * D + 16 * p);
         if (it.q_row0 + row < a.Tq) __builtin_nontemporal_store(w, dst(row));
       }
+    }
+  }
+
+  // ---- key splits -------------------------------------------------------------------------
+  // Partials of one wave: its accumulators as the lanes hold them (float4 rq of column block dt of
+  // lane l at ((4 dt + rq) * 64 + l) * 4), then the row references and row sums of its 32 rows.
+  static constexpr int PART_WORDS = QT * D + 2 * QT;
+  static __device__ __forceinline__ void store_partial(const PrefillArgs& a, const f32x16 (&O)[D / 32], float m_ref,
+                                                       float l_run, int slot, int lane) {
+    float* p = a.part + (int64_t)slot * PART_WORDS;
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+      for (int rq = 0; rq < 4; ++rq)
+        *reinterpret_cast<f32x4*>(p + ((4 * dt + rq) * 64 + lane) * 4) =
+            f32x4{O[dt][4 * rq], O[dt][4 * rq + 1], O[dt][4 * rq + 2], O[dt][4 * rq + 3]};
+    const float lt = halves_sum(l_run);
+    if (lane < QT) {
+      p[QT * D + lane] = m_ref;
+      p[QT * D + QT + lane] = lt;
+    }
+  }
+
+  // Merges the splits of one column block (32 columns) of one wave of an item: wave index
+  // ((item * NW) + w) * (D / 32) + dt.  Four splits' partials load at a time, each load a whole KiB.
+  static __device__ void combine(const PrefillArgs& a, int n_waves) {
+    const int lane = threadIdx.x & 63;
+    const int x = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (x >= n_waves) return;
+    const int dt = x % (D / 32), iw = x / (D / 32), w = iw % NW, item = iw / NW;
+    int qt, r, hs, b;
+    decode_item_uniform(a, item * a.splits, qt, r, hs, b);
+    const int l32 = lane & 31, g = lane >> 5;
+    const int64_t split_stride = (int64_t)NW * PART_WORDS;
+    const float* p0 = a.part + ((int64_t)item * a.splits * NW + w) * PART_WORDS;
+    constexpr int CH = 4;
+    float M = -__builtin_inff(), L = 0.f;
+    f32x4 acc[4] = {f32x4{}, f32x4{}, f32x4{}, f32x4{}};
+    for (int s0 = 0; s0 < a.splits; s0 += CH) {
+      float m[CH], l[CH];
+      f32x4 v[CH][4];
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        const float* p = p0 + min(s0 + i, a.splits - 1) * split_stride;  // past the last: a repeat, not used
+        m[i] = p[QT * D + l32];
+        l[i] = p[QT * D + QT + l32];
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq) v[i][rq] = *reinterpret_cast<const f32x4*>(p + ((4 * dt + rq) * 64 + lane) * 4);
+      }
+      float Mc = M;
+#pragma unroll
+      for (int i = 0; i < CH; ++i)
+        if (s0 + i < a.splits) Mc = fmaxf(Mc, m[i]);
+      const float Mu = Mc == -__builtin_inff() ? 0.f : Mc;
+      const float f0 = fast_exp2(M - Mu);  // 0 while nothing has been merged
+      L *= f0;
+#pragma unroll
+      for (int rq = 0; rq < 4; ++rq) acc[rq] *= f0;
+#pragma unroll
+      for (int i = 0; i < CH; ++i)
+        if (s0 + i < a.splits) {
+          const float f = fast_exp2(m[i] - Mu);
+          L += f * l[i];
+#pragma unroll
+          for (int rq = 0; rq < 4; ++rq) acc[rq] += f * v[i][rq];
+        }
+      M = Mc;
+    }
+    const float inv = L > 0.f ? 1.f / L : 1.f;
+    const int row = qt * QTILE + QT * (w / HW) + l32;
+    elem_t* ob = a.o + b * a.o_sb + (r * a.heads_per_row + hs * HW + w % HW) * a.o_sh;
+    // Lane (l32, g) holds columns 8 rq + 4 g .. + 3 of the block; after the swaps lane g holds all 8 of
+    // rq = 2 h + g, one 16-byte store.
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      u32x4 o;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const uint32_t x0 = E::pack2f(acc[2 * h][2 * e] * inv, acc[2 * h][2 * e + 1] * inv);
+        const uint32_t x1 = E::pack2f(acc[2 * h + 1][2 * e] * inv, acc[2 * h + 1][2 * e + 1] * inv);
+        const auto sw = __builtin_amdgcn_permlane32_swap(x0, x1, false, false);
+        o[e] = sw[0];
+        o[2 + e] = sw[1];
+      }
+      if (row < a.Tq) *reinterpret_cast<u32x4*>(ob + (int64_t)row * a.o_st + 32 * dt + 8 * (2 * h + g)) = o;
     }
   }
 
@@ -1068,7 +1164,7 @@ struct Prefill {
   template <bool LOOK>
   static __device__ __forceinline__ void item_pipelined(const PrefillArgs& a, int qt, int r, int hs, int b,
                                                         char* sKV, char* sQ, int32_t* s_row, int32_t* s_mask,
-                                                        const Look* lk, int& vb_first) {
+                                                        const Look* lk, int& vb_first, int item_id) {
     char* sK = sKV;
     char* sV = sKV + NBK * TILE_BYTES;
     const int lane = threadIdx.x & 63;
@@ -1116,6 +1212,12 @@ struct Prefill {
     // wave has passed the barrier below: the K buffers were last read before the previous
     // item's last barrier, and its last step reads only the other two V buffers.
     TileQueue q = queue_begin(a, it);
+    if constexpr (KS) {  // key tiles [n x / splits, n (x + 1) / splits) of the n before the limit
+      const int x = item_id - (int)fast_div((uint32_t)item_id, (uint32_t)a.splits, a.mul_splits) * a.splits;
+      const int64_t n = kt_limit(a, it) + 1;
+      q.kt_lo = (int)(n * x / a.splits);
+      q.kt_hi = (int)(n * (x + 1) / a.splits) - 1;
+    }
     int kt_cur = 0, kt_nxt = 0;
     uint32_t m_cur = 0u, m_nxt = 0u;
     bool has_cur = queue_pop(a, it, s_row, s_mask, q, kt_cur, m_cur);
@@ -1375,7 +1477,10 @@ struct Prefill {
     }
     tl_stamp(TL_LAST);
     // O is staged in the wave's own Q slot (Q is in registers): no other wave touches it.
-    epilogue(a, it, b, O, l_run, sQw, lane);
+    if constexpr (KS)
+      store_partial(a, O, m_ref, l_run, item_id * NW + wave, lane);
+    else
+      epilogue(a, it, b, O, l_run, sQw, lane);
     tl_stamp(TL_EPILOGUE);
     tl_count(TL_ITEMS);
   }
@@ -1385,6 +1490,7 @@ struct Prefill {
   // tile together; with it: row by row (s_row_rank), latest query tiles first within a row.
   static __device__ __forceinline__ void decode_item(const PrefillArgs& a, int v, int& qt, int& r, int& hs, int& b) {
     uint32_t rem;
+    if constexpr (KS) v = (int)fast_div((uint32_t)v, (uint32_t)a.splits, a.mul_splits);
     if (a.row_order && v >= a.head_items) {
       const uint32_t w = (uint32_t)(v - a.head_items);
       const uint32_t k = fast_div(w, (uint32_t)a.per_group, a.mul_group);
@@ -1443,7 +1549,7 @@ struct Prefill {
     if constexpr (PIPE)
     {
       int vb_first = 0;
-      item_pipelined<false>(a, qt, r, hs, b, sKV, sQ, s_row, s_mask, nullptr, vb_first);
+      item_pipelined<false>(a, qt, r, hs, b, sKV, sQ, s_row, s_mask, nullptr, vb_first, v);
     }
     else
       item<false>(a, qt, r, hs, b, sKV, s_ml, s_row, s_mask, nullptr);
@@ -1542,7 +1648,7 @@ struct Prefill {
       int32_t* row = s_row + (i & 1) * RC;
       int32_t* mask = SUB ? s_mask + (i & 1) * RC : s_mask;
       if constexpr (PIPE)
-        item_pipelined<true>(a, qt, r, hs, b, sKV, sQ, row, mask, &lk, vb_first);
+        item_pipelined<true>(a, qt, r, hs, b, sKV, sQ, row, mask, &lk, vb_first, v);
       else
         item<true>(a, qt, r, hs, b, sKV, s_ml, row, mask, &lk);
     }
@@ -1555,7 +1661,7 @@ struct Prefill {
     // Row caches: two for the persistent loop (this item and the next one).
     __shared__ int32_t s_row[2 * RC];
     __shared__ int32_t s_mask[SUB ? 2 * RC : 1];  // sub-block masks of the cached rows
-    const int n_items = a.ntq * a.R * a.B * a.head_splits;
+    const int n_items = a.ntq * a.R * a.B * a.head_splits * (KS ? a.splits : 1);
 
     if (!a.claims) {
       // One workgroup per item.  Consecutive workgroups go to the 8 XCDs in turn; chunks of
@@ -1614,6 +1720,17 @@ void prefill_kernel(PrefillArgs a) {
   Prefill<BF16, D, HW, NS, SUB>::run(a);
 }
 
+// Four-head workgroups with key splits, and the merge of their partials.
+template <bool BF16, int D, bool SUB>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
+void prefill_split_kernel(PrefillArgs a) {
+  Prefill<BF16, D, 4, 1, SUB, false, true>::run(a);
+}
+template <bool BF16, int D>
+__global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a, int n_waves) {
+  Prefill<BF16, D, 4, 1, false, false, true>::combine(a, n_waves);
+}
+
 // The timeline instantiation of the persistent four-head kernel (head dim 128, blocks of 64 or 128).
 template <bool BF16>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
@@ -1660,6 +1777,21 @@ template <bool BF16, int D, int HW, int NS>
 static hipError_t launch_hw(const PrefillArgs& a, int64_t n_items, int64_t item_grid, hipStream_t s) {
   return a.sub_log2 ? launch_sub<BF16, D, HW, NS, true>(a, n_items, item_grid, s)
                     : launch_sub<BF16, D, HW, NS, false>(a, n_items, item_grid, s);
+}
+
+template <bool BF16, int D>
+static hipError_t launch_split(const PrefillArgs& a, int64_t items, hipStream_t s) {
+  const dim3 grid((unsigned)(items * a.splits));
+  if (a.sub_log2)
+    hipLaunchKernelGGL((prefill_split_kernel<BF16, D, true>), grid, dim3(512), 0, s, a);
+  else
+    hipLaunchKernelGGL((prefill_split_kernel<BF16, D, false>), grid, dim3(512), 0, s, a);
+  const hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  const int64_t n_waves = items * 8 * (D / 32);
+  hipLaunchKernelGGL((prefill_combine_kernel<BF16, D>), dim3((unsigned)ceil_div(n_waves, 4)), dim3(256), 0, s, a,
+                     (int)n_waves);
+  return hipGetLastError();
 }
 
 template <bool BF16, int D>
@@ -1713,6 +1845,31 @@ static Shape choose_shape(int T_q, int T_k, int rows, int B, int heads_per_row) 
   return {hw, waves <= 4 * cus ? 2 : 1};
 }
 
+// Key splits of a four-head launch (1: none).  One workgroup per item leaves CUs idle when items are
+// few and long (a chunk of a prompt over a cached prefix): their key tiles are then divided over as
+// many workgroups as there are CUs, at least eight key tiles each.  pairs_stride is at least a row's
+// entries, so it bounds the tiles per query tile (an entry of a finer schedule is counted as the share
+// of a tile that it fills): below 32 of them the partials and the merge would cost what the division
+// gains.  Measured (32 heads on 4,000 keys and the queries' own, us, one workgroup or slices against
+// key splits): 16 queries 50.1 / 26.7, 256 queries 55.6 / 36.7, 512 queries 62.7 / 54.0, 1,000 queries 114.7 / 95.2
+// (the 34 MB of partials and the merge are about 15 of them).
+static int choose_splits(int T_q, int T_k, int rows, int B, int heads_per_row, int block_size, int64_t pairs_stride) {
+  if (heads_per_row % 4) return 1;
+  const int64_t items = ceil_div(T_q, QTILE) * rows * (int64_t)B * (heads_per_row / 4);
+  const int64_t tiles = ceil_div(T_k, KT);
+  if (items == 0 || 2 * items > num_cus() || tiles < 32) return 1;
+  const int64_t entries = pairs_stride / ceil_div(T_q, std::max(block_size, QTILE));  // per query block
+  const int64_t sub = block_size < KT ? KT / block_size : 1, per_entry = block_size > KT ? block_size / KT : 1;
+  if (entries * per_entry < 32 * sub * sub) return 1;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(num_cus() / items, tiles / 8), 32));
+}
+
+static int64_t split_bytes(int T_q, int rows, int B, int heads_per_row, int D, int splits) {
+  if (splits <= 1) return 0;
+  const int64_t items = ceil_div(T_q, QTILE) * rows * (int64_t)B * (heads_per_row / 4);
+  return items * splits * 8 * (QT * D + 2 * QT) * (int64_t)sizeof(float);
+}
+
 static int prefill_impl(const char* fn, int dtype,
                         const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st,
                         const void* k, int64_t k_sb, int64_t k_sh, int64_t k_st,
@@ -1725,6 +1882,7 @@ static int prefill_impl(const char* fn, int dtype,
                         int B, int Hq, int Hkv, int T_q, int T_k, int D,
                         int block_size, int q_offset, float sm_scale,
                         void* workspace, int64_t workspace_bytes,
+                        void* partials, int64_t partials_bytes,
                         void* stream,
                         unsigned long long* timeline, int64_t timeline_words) {
   clear_error();
@@ -1776,8 +1934,15 @@ static int prefill_impl(const char* fn, int dtype,
   a.sub_log2 = block_size == 16 ? 4 : block_size == 32 ? 5 : 0;
   a.R = csr_rows;
   a.heads_per_row = Hq / csr_rows;
-  const Shape shape = timeline ? Shape{(a.heads_per_row % 4 == 0) ? 4 : 1, 1}
-                               : choose_shape(T_q, T_k, csr_rows, B, a.heads_per_row);
+  a.splits = 1;
+  if (partials && workspace && !timeline) {
+    const int n = choose_splits(T_q, T_k, csr_rows, B, a.heads_per_row, block_size, pairs_stride);
+    if (partials_bytes >= split_bytes(T_q, csr_rows, B, a.heads_per_row, D, n)) a.splits = n;
+  }
+  a.mul_splits = div_mul((uint32_t)a.splits);
+  a.part = static_cast<float*>(partials);
+  const Shape shape = timeline || a.splits > 1 ? Shape{(a.heads_per_row % 4 == 0) ? 4 : 1, 1}
+                                               : choose_shape(T_q, T_k, csr_rows, B, a.heads_per_row);
   const int hw = shape.hw, ns = shape.ns;
   a.head_splits = a.heads_per_row / hw;
   a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.Tq = T_q; a.Tk = T_k;
@@ -1844,6 +2009,9 @@ static int prefill_impl(const char* fn, int dtype,
     else
       hipLaunchKernelGGL((prefill_timeline_kernel<false>), dim3(grid), dim3(512), 0, s, a);
     err = hipGetLastError();
+  } else if (a.splits > 1) {
+    err = D == 128 ? (bf16 ? launch_split<true, 128>(a, n_items, s) : launch_split<false, 128>(a, n_items, s))
+                   : (bf16 ? launch_split<true, 64>(a, n_items, s) : launch_split<false, 64>(a, n_items, s));
   } else if (D == 128)
     err = bf16 ? launch_d<true, 128>(a, hw, ns, n_items, item_grid, s) : launch_d<false, 128>(a, hw, ns, n_items, item_grid, s);
   else
@@ -1870,7 +2038,36 @@ extern "C" int sa_prefill(int dtype,
   return sa::prefill_impl("sa_prefill", dtype, q, q_sb, q_sh, q_st, k, k_sb, k_sh, k_st, v, v_sb, v_sh, v_st,
                           o, o_sb, o_sh, o_st, pairs, pairs_stride, offsets, offsets_stride, tile_masks,
                           tile_masks_stride, csr_rows, nqb, B, Hq, Hkv, T_q, T_k, D, block_size, q_offset,
-                          sm_scale, workspace, workspace_bytes, stream, nullptr, 0);
+                          sm_scale, workspace, workspace_bytes, nullptr, 0, stream, nullptr, 0);
+}
+
+extern "C" int sa_prefill_split(int dtype,
+                                const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st,
+                                const void* k, int64_t k_sb, int64_t k_sh, int64_t k_st,
+                                const void* v, int64_t v_sb, int64_t v_sh, int64_t v_st,
+                                void* o, int64_t o_sb, int64_t o_sh, int64_t o_st,
+                                const int32_t* pairs, int64_t pairs_stride,
+                                const int32_t* offsets, int64_t offsets_stride,
+                                const int32_t* tile_masks, int64_t tile_masks_stride,
+                                int csr_rows, int nqb,
+                                int B, int Hq, int Hkv, int T_q, int T_k, int D,
+                                int block_size, int q_offset, float sm_scale,
+                                void* workspace, int64_t workspace_bytes,
+                                void* partials, int64_t partials_bytes,
+                                void* stream) {
+  return sa::prefill_impl("sa_prefill_split", dtype, q, q_sb, q_sh, q_st, k, k_sb, k_sh, k_st, v, v_sb, v_sh, v_st,
+                          o, o_sb, o_sh, o_st, pairs, pairs_stride, offsets, offsets_stride, tile_masks,
+                          tile_masks_stride, csr_rows, nqb, B, Hq, Hkv, T_q, T_k, D, block_size, q_offset,
+                          sm_scale, workspace, workspace_bytes, partials, partials_bytes, stream, nullptr, 0);
+}
+
+extern "C" int64_t sa_prefill_partial_bytes(int csr_rows, int B, int Hq, int T_q, int T_k, int D, int block_size,
+                                            int64_t pairs_stride) {
+  using namespace sa;
+  if (csr_rows < 1 || B < 1 || Hq < 1 || Hq % csr_rows || T_q < 1 || T_k < 1 || (D != 64 && D != 128) || block_size < 1)
+    return 0;
+  const int hpr = Hq / csr_rows;
+  return split_bytes(T_q, csr_rows, B, hpr, D, choose_splits(T_q, T_k, csr_rows, B, hpr, block_size, pairs_stride));
 }
 
 extern "C" int sa_prefill_timeline(int dtype,
@@ -1891,7 +2088,7 @@ extern "C" int sa_prefill_timeline(int dtype,
   return sa::prefill_impl("sa_prefill_timeline", dtype, q, q_sb, q_sh, q_st, k, k_sb, k_sh, k_st, v, v_sb, v_sh,
                           v_st, o, o_sb, o_sh, o_st, pairs, pairs_stride, offsets, offsets_stride, nullptr, 0,
                           csr_rows, nqb, B, Hq, Hkv, T_q, T_k, D, block_size, q_offset, sm_scale, workspace,
-                          workspace_bytes, stream, reinterpret_cast<unsigned long long*>(timeline),
+                          workspace_bytes, nullptr, 0, stream, reinterpret_cast<unsigned long long*>(timeline),
                           timeline_words);
 }
 

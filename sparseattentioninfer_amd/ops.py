@@ -303,7 +303,8 @@ def universal_sparse_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     # `held` keeps the schedule tensors alive until the launch is enqueued: freed earlier,
     # their memory could be handed to an allocation (the workspace below) ahead of the kernel.
     *held, sched, nqb_k = _schedule_args(pairs, offsets, block_size, tiles)
-    status = lib.sa_prefill(
+    part = _partials(sched[1], R, B, Hq, T_q, T_k, D, block_size, q.device)
+    status = lib.sa_prefill_split(
         _DTYPES[q.dtype],
         q.data_ptr(), q.stride(0), q.stride(1), q.stride(2),
         k.data_ptr(), k.stride(0), k.stride(1), k.stride(2),
@@ -311,14 +312,26 @@ def universal_sparse_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         out.data_ptr(), out.stride(0), out.stride(1), out.stride(2),
         *sched,
         R, nqb_k, B, Hq, Hkv, T_q, T_k, D, block_size, int(q_offset), sm_scale,
-        *_ws_args(_prefill_workspace(q)), _stream(q))
-    del held   # enqueued: a later reuse of this memory is ordered after the kernel on the stream
+        *_ws_args(_prefill_workspace(q)), *_partial_args(part), _stream(q))
+    del held, part   # enqueued: a later reuse of this memory is ordered after the kernel on the stream
     _lib.check("sa_prefill", status)
     return out
 
 
 def _ws_args(ws: torch.Tensor):
     return ws.data_ptr(), ws.numel() * ws.element_size()
+
+
+def _partials(pairs_stride: int, R: int, B: int, Hq: int, T_q: int, T_k: int, D: int, block_size: int,
+              device) -> torch.Tensor | None:
+    """Buffer for the partial results of a prefill launch that divides its keys over workgroups, or
+    None where the launch does not."""
+    n = int(_lib.load().sa_prefill_partial_bytes(R, B, Hq, T_q, T_k, D, block_size, pairs_stride))
+    return torch.empty(n, dtype=torch.uint8, device=device) if n else None
+
+
+def _partial_args(part: torch.Tensor | None):
+    return (None, 0) if part is None else (part.data_ptr(), part.numel())
 
 
 def _kv_strides(k, v, name):
@@ -467,6 +480,7 @@ def prepare_prefill(q, k, v, block_pairs, block_pair_offsets, block_size, *, out
     sp, so, sm, sched, nqb_k = _schedule_args(pairs, offsets, block_size, None)
     if out is None:
         out = torch.empty(B, Hq, T_q, D, dtype=q.dtype, device=q.device)
+    part = _partials(sched[1], R, B, Hq, T_q, T_k, D, block_size, q.device)
     args = [
         _DTYPES[q.dtype],
         q.data_ptr(), q.stride(0), q.stride(1), q.stride(2),
@@ -475,8 +489,8 @@ def prepare_prefill(q, k, v, block_pairs, block_pair_offsets, block_size, *, out
         out.data_ptr(), out.stride(0), out.stride(1), out.stride(2),
         *sched,
         R, nqb_k, B, Hq, Hkv, T_q, T_k, D, block_size, T_k - T_q,
-        1.0 / math.sqrt(D), *_ws_args(_prefill_workspace(q)), _stream(q)]
-    return PreparedLaunch("sa_prefill", args, (q, k, v, pairs, offsets, sp, so, sm), out)
+        1.0 / math.sqrt(D), *_ws_args(_prefill_workspace(q)), *_partial_args(part), _stream(q)]
+    return PreparedLaunch("sa_prefill_split", args, (q, k, v, pairs, offsets, sp, so, sm, part), out)
 
 
 TIMELINE_RECORD_WORDS = 36    # words per workgroup written by sa_prefill_timeline
