@@ -18,9 +18,8 @@
 //       qa (clipped to NKB - 1) is kept; nothing above it.
 //     - Seeded BigBird: the global prefix, the window (trailing {qa-w+1..qa} or centred
 //       {qa-w/2..qa+w/2}) and the diagonal, causal-truncated, plus counts[row] random blocks:
-//       the eligible (causal, not already kept) blocks with the smallest (draw, kb).  A first
-//       kernel writes everything but the random picks (one thread per 16 bytes); a second
-//       kernel, one wave per (row, query block), takes the counts[row] smallest draws.
+//       the eligible (causal, not already kept) blocks with the smallest (draw, kb).  One wave per
+//       (row, query block) writes the kept blocks and takes the counts[row] smallest draws.
 #include <algorithm>
 
 #include "sa_common.h"
@@ -60,7 +59,7 @@ __device__ __forceinline__ uint64_t block_draw(uint64_t seed, uint64_t stream, i
 }
 
 // ---- byte-parallel fill ------------------------------------------------------------------
-enum FillKind : int { FILL_BIGBIRD_HASH = 0, FILL_SEEDED_BASE = 1, FILL_BERNOULLI = 2 };
+enum FillKind : int { FILL_BIGBIRD_HASH = 0, FILL_BERNOULLI = 1 };
 
 struct FillArgs {
   uint8_t* mask;
@@ -72,8 +71,6 @@ struct FillArgs {
   int head_base;             // hash head of row `row` = head_base + row
   int hash_blocks;           // num_blocks in the hash
   int dense_last;            // last query block keeps every block
-  // seeded BigBird base
-  int window, global_blocks, centred;
   // Bernoulli
   uint64_t seed;
   uint64_t threshold;        // keep iff (draw >> 11) < threshold
@@ -101,12 +98,6 @@ __device__ __forceinline__ bool fill_bit(const FillArgs& a, int row, int i, int 
   const int qa = min(a.qbo + i, a.nkb - 1);  // causal limit of the query block
   if (kb > qa) return false;
   if (kb == qa) return true;
-  if (a.kind == FILL_SEEDED_BASE) {
-    if (kb < a.global_blocks) return true;
-    const int lo = a.centred ? qa - a.window / 2 : qa - a.window + 1;
-    const int hi = a.centred ? qa + a.window / 2 : qa;
-    return kb >= lo && kb <= hi;
-  }
   return (block_draw(a.seed, 2, row, qa, kb) >> 11) < a.threshold;  // FILL_BERNOULLI
 }
 
@@ -130,7 +121,7 @@ __global__ __launch_bounds__(PAT_THREADS) void block_mask_fill_kernel(FillArgs a
   }
 }
 
-// ---- seeded random picks -----------------------------------------------------------------
+// ---- seeded BigBird --------------------------------------------------------------------------
 struct PickArgs {
   uint8_t* mask;
   int64_t mask_sr, mask_sq;
@@ -144,10 +135,19 @@ __device__ __forceinline__ bool less_key(uint64_t u, int kb, uint64_t v, int kc)
   return u < v || (u == v && kb < kc);
 }
 
-// One wave per (row, query block); PAT_THREADS / 64 of them per workgroup.  Round j takes the
+// One wave per (row, query block); PAT_THREADS / 64 of them per workgroup.  The wave writes the row's
+// window, global and diagonal blocks, 16 bytes per lane, then the picks: a pick's byte is stored by the
+// lane that wrote its 16, so the two stores are in order.  Round j takes the
 // eligible block with the smallest (draw, kb) greater than round j - 1's, so the picks are the
 // counts[row] smallest keys, found without replacement and independent of lane timing.
+// Bound by the draws (a Philox of ten rounds of two 64 x 64-bit products each): every draw is made
+// once and kept in LDS for the rounds.  8 rows of 512 query blocks, 3 picks: 41 us with the draws
+// made anew in every round and 6 us for a fill kernel before it, 25 us now for both.  Rows of more than PICK_CACHE blocks, whose draws do not
+// fit, still make them in every round.
+constexpr int PICK_CACHE = 1024;  // draws of a wave kept in LDS (8 KiB)
+
 __global__ __launch_bounds__(PAT_THREADS) void block_mask_pick_kernel(PickArgs a) {
+  __shared__ uint64_t s_draw[PAT_THREADS / 64][PICK_CACHE];
   const int lane = threadIdx.x & 63;
   const int64_t wid = (int64_t)blockIdx.x * (PAT_THREADS / 64) + (threadIdx.x >> 6);
   if (wid >= (int64_t)a.rows * a.nqb) return;
@@ -158,14 +158,36 @@ __global__ __launch_bounds__(PAT_THREADS) void block_mask_pick_kernel(PickArgs a
   const int hi = a.centred ? qa + a.window / 2 : qa;
   uint8_t* m = a.mask + row * a.mask_sr + (int64_t)i * a.mask_sq;
   const int count = a.counts[row];
+  uint64_t* draws = s_draw[threadIdx.x >> 6];
+  const bool keep = qa <= PICK_CACHE;
+  // eligible: causal, not global / window / diagonal
+  auto eligible = [&](int kb) { return kb >= a.global_blocks && (kb < lo || kb > hi); };
+  for (int c = lane; c < (int)(a.mask_sq / 16); c += 64) {
+    uint32_t w[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      uint32_t v = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int kb = 16 * c + 4 * q + e;
+        v |= (uint32_t)(kb <= qa && (kb == qa || !eligible(kb))) << (8 * e);
+      }
+      w[q] = v;
+    }
+    *reinterpret_cast<u32x4*>(m + 16 * c) = u32x4{w[0], w[1], w[2], w[3]};
+  }
+  // A lane reads only what it wrote itself.
+  if (keep && count > 0)
+    for (int kb = lane; kb < qa; kb += 64)
+      if (eligible(kb)) draws[kb] = block_draw(a.seed, 1, row, qa, kb);
   uint64_t prev_u = 0;
   int prev_kb = -1;  // (0, -1) precedes every key
   for (int j = 0; j < count; ++j) {
     uint64_t best_u = ~0ull;
     int best_kb = 0x7fffffff;
-    for (int kb = lane; kb < qa; kb += 64) {  // eligible: causal, not global / window / diagonal
-      if (kb < a.global_blocks || (kb >= lo && kb <= hi)) continue;
-      const uint64_t u = block_draw(a.seed, 1, row, qa, kb);
+    for (int kb = lane; kb < qa; kb += 64) {
+      if (!eligible(kb)) continue;
+      const uint64_t u = keep ? draws[kb] : block_draw(a.seed, 1, row, qa, kb);
       if (less_key(prev_u, prev_kb, u, kb) && less_key(u, kb, best_u, best_kb)) {
         best_u = u;
         best_kb = kb;
@@ -181,7 +203,7 @@ __global__ __launch_bounds__(PAT_THREADS) void block_mask_pick_kernel(PickArgs a
       }
     }
     if (best_kb == 0x7fffffff) break;  // fewer eligible blocks than count: all taken
-    if (lane == 0) m[best_kb] = 1;
+    if (lane == (best_kb / 16) % 64) m[best_kb] = 1;
     prev_u = best_u;
     prev_kb = best_kb;
   }
@@ -240,12 +262,6 @@ extern "C" int sa_seeded_bigbird_block_mask(uint8_t* mask, int64_t mask_row_stri
   if (rows && nqb && !random_counts) return set_error(SA_E_NULL, "%s: NULL random_counts", name);
   if (q_block_offset < 0 || window < 0 || global_blocks < 0)
     return set_error(SA_E_SHAPE, "%s: negative offset / window / global", name);
-  FillArgs a{};
-  a.mask = mask; a.mask_sr = mask_row_stride; a.mask_sq = mask_qb_stride;
-  a.rows = rows; a.nqb = nqb; a.nkb = nkb; a.qbo = q_block_offset;
-  a.kind = FILL_SEEDED_BASE;
-  a.window = window; a.global_blocks = global_blocks; a.centred = centred != 0;
-  if (int rc = fill_launch(a, stream, name)) return rc;
   const int64_t waves = (int64_t)rows * nqb;
   if (waves == 0) return 0;
   PickArgs p{};
