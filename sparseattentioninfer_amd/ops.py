@@ -23,8 +23,14 @@ from .patterns.base import kv_block_list_to_pairs
 _DTYPES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16}
 
 
+# The calling thread's current stream of a device, as the pointer itself: the stream object that
+# torch.cuda.current_stream builds around it costs 3-4 us a call, a fifth of a small decode call.
+_raw_stream = torch._C._cuda_getCurrentRawStream if hasattr(torch._C, "_cuda_getCurrentRawStream") else \
+    (lambda index: torch.cuda.current_stream(index).cuda_stream)
+
+
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.device.index)
 
 
 _PREFILL_WS: dict = {}
@@ -127,20 +133,27 @@ def block_mask_to_csr_gpu(block_active: torch.Tensor) -> tuple[torch.Tensor, tor
     m = block_active.to(torch.uint8) if block_active.dtype != torch.uint8 else block_active
     if m.stride(2) != 1:
         m = m.contiguous()
+    return csr_of_mask(m)[:2]
+
+
+def csr_of_mask(m: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor, list]:
+    """``(pairs, offsets, entries per row)`` of a uint8 block mask on the GPU whose key blocks are
+    contiguous; the entries are what the one read between the passes brings to the host."""
+    name = "block_mask_to_csr"
     R, nqb, nkb = m.shape
     dev = m.device
     offsets = torch.empty(R, nqb + 1, dtype=torch.int32, device=dev)
-    nnz = torch.empty(R, dtype=torch.int32, device=dev)
+    nnz = torch.empty(R + 1, dtype=torch.int32, device=dev)     # and the write pass's status word (never set)
     lib = _lib.load()
     args = (m.data_ptr(), m.stride(0), m.stride(1), R, nqb, nkb, offsets.data_ptr(), offsets.stride(0),
             nnz.data_ptr())
     _lib.check(name, lib.sa_block_mask_to_csr(*args, None, 0, 0, None, _stream(m)))
-    width = max(1, int(nnz.max().item())) if R else 1
+    counts = nnz.tolist()[:R] if R else []
+    width = max(1, *counts) if R else 1
     pairs = torch.empty(R, width, dtype=torch.int32, device=dev)
-    status = torch.zeros(1, dtype=torch.int32, device=dev)
     _lib.check(name, lib.sa_block_mask_to_csr(*args, pairs.data_ptr(), pairs.stride(0), width,
-                                              status.data_ptr(), _stream(m)))
-    return pairs, offsets
+                                              nnz[R:].data_ptr(), _stream(m)))
+    return pairs, offsets, counts
 
 
 def _mask_buffer(rows: int, nqb: int, nkb: int, device) -> torch.Tensor:
@@ -181,11 +194,14 @@ def seeded_bigbird_block_mask_gpu(rows: int, nqb: int, nkb: int, *, window: int,
     """Seeded BigBird rows on Philox4x64-10 (see ``include/sparse_attn.h``), ``[R, NQB, NKB]`` uint8."""
     _require(window_align in ("trailing", "centred"), f"window_align must be 'trailing' or 'centred', got {window_align!r}")
     device = torch.device(device)
-    counts = torch.as_tensor(random_blocks, dtype=torch.int32).reshape(-1)
-    if counts.numel() == 1:
-        counts = counts.expand(rows)
-    _require(counts.numel() == rows, f"random_blocks has {counts.numel()} entries for {rows} rows")
-    counts = counts.contiguous().to(device)
+    if isinstance(random_blocks, int):      # filled on the device: a copy from the host would wait for it
+        counts = torch.full((rows,), random_blocks, dtype=torch.int32, device=device)
+    else:
+        counts = torch.as_tensor(random_blocks, dtype=torch.int32).reshape(-1)
+        if counts.numel() == 1:
+            counts = counts.expand(rows)
+        _require(counts.numel() == rows, f"random_blocks has {counts.numel()} entries for {rows} rows")
+        counts = counts.contiguous().to(device)
     buf = _mask_buffer(rows, nqb, nkb, device)
     return _mask_call("sa_seeded_bigbird_block_mask", _lib.load().sa_seeded_bigbird_block_mask, buf, rows, nqb,
                       nkb, int(q_block_offset), int(window), int(global_blocks), int(window_align == "centred"),
@@ -223,6 +239,13 @@ def _require(cond: bool, msg: str) -> None:
 
 
 def _check_qkv(q, k, v, name):
+    """Validates q, k and v.  One test of everything first: a call that passes formats no message."""
+    qs, ks = q.shape, k.shape
+    if (q.is_cuda and k.is_cuda and v.is_cuda and k.device == q.device and v.device == q.device
+            and q.dtype in _DTYPES and k.dtype == q.dtype and v.dtype == q.dtype
+            and len(qs) == 4 and len(ks) == 4 and ks == v.shape and qs[0] == ks[0] and qs[3] == ks[3]
+            and qs[1] % ks[1] == 0 and q.stride(3) == 1 and k.stride(3) == 1 and v.stride(3) == 1):
+        return
     _require(q.is_cuda, f"{name} requires CUDA tensors")
     _require(k.is_cuda and v.is_cuda and k.device == q.device and v.device == q.device,
              f"{name}: q, k and v must be on the same GPU")
@@ -255,16 +278,19 @@ def universal_sparse_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     _check_qkv(q, k, v, name)
     B, Hq, T_q, D = q.shape
     Hkv, T_k = k.shape[1], k.shape[2]
-    _require(block_size >= 16 and (block_size & (block_size - 1)) == 0,
-             "block_size must be a power of 2 and >= 16")
-    _require(block_pairs.dtype == torch.int32, "block_pairs must be int32")
-    _require(block_pair_offsets.dtype == torch.int32, "block_pair_offsets must be int32")
     R = block_pairs.size(0)
-    _require(R in (Hq, Hkv), f"block_pairs head dim {R} != H={Hq} (or KV heads {Hkv})")
-    _require(block_pair_offsets.size(0) == R,
-             f"block_pair_offsets head dim {block_pair_offsets.size(0)} != H={R}")
-    _require(block_pairs.device == q.device and block_pair_offsets.device == q.device,
-             f"{name}: CSR tensors must be on the GPU of q")
+    if not (block_size >= 16 and (block_size & (block_size - 1)) == 0 and block_pairs.dtype == torch.int32
+            and block_pair_offsets.dtype == torch.int32 and (R == Hq or R == Hkv) and block_pair_offsets.size(0) == R
+            and block_pairs.device == q.device and block_pair_offsets.device == q.device):
+        _require(block_size >= 16 and (block_size & (block_size - 1)) == 0,
+                 "block_size must be a power of 2 and >= 16")
+        _require(block_pairs.dtype == torch.int32, "block_pairs must be int32")
+        _require(block_pair_offsets.dtype == torch.int32, "block_pair_offsets must be int32")
+        _require(R in (Hq, Hkv), f"block_pairs head dim {R} != H={Hq} (or KV heads {Hkv})")
+        _require(block_pair_offsets.size(0) == R,
+                 f"block_pair_offsets head dim {block_pair_offsets.size(0)} != H={R}")
+        _require(block_pairs.device == q.device and block_pair_offsets.device == q.device,
+                 f"{name}: CSR tensors must be on the GPU of q")
     pairs = block_pairs.contiguous()
     offsets = block_pair_offsets.contiguous()
     nqb = offsets.size(1) - 1
@@ -274,7 +300,8 @@ def universal_sparse_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     out = torch.empty(B, Hq, T_q, D, dtype=q.dtype, device=q.device)
     lib = _lib.load()
     if T_q == 1 and q_offset == T_k - 1:
-        _require(nqb == 1, f"{name}: decode expects one CSR query block, got {nqb}")
+        if nqb != 1:
+            raise AssertionError(f"{name}: decode expects one CSR query block, got {nqb}")
         # Lists of 1,024 keys and more are split over workgroups: unsplit, a row's list is read by one CU
         # (4 sequences of 8,191 tokens, 32 heads, 8 KV heads: 137 us; split by 8, 27 us).  Shorter ones are
         # not: the partials and the combine cost an eager call 5 us of launching (256 keys of 8 heads: 15 us
@@ -296,10 +323,10 @@ def universal_sparse_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
             splits, ws.data_ptr() if ws is not None else None, ws_bytes, _stream(q))
         _lib.check("sa_decode", status)
         return out
-    _require(block_size <= 128, f"{name}: block_size {block_size} not supported by the "
-             "gfx950 prefill kernel (16, 32, 64, 128)")
-    _require(nqb == -(-T_q // block_size),
-             f"{name}: {nqb} CSR query blocks but T_q={T_q} needs {-(-T_q // block_size)}")
+    if block_size > 128 or nqb != -(-T_q // block_size):
+        _require(block_size <= 128, f"{name}: block_size {block_size} not supported by the "
+                 "gfx950 prefill kernel (16, 32, 64, 128)")
+        _require(False, f"{name}: {nqb} CSR query blocks but T_q={T_q} needs {-(-T_q // block_size)}")
     # `held` keeps the schedule tensors alive until the launch is enqueued: freed earlier,
     # their memory could be handed to an allocation (the workspace below) ahead of the kernel.
     *held, sched, nqb_k = _schedule_args(pairs, offsets, block_size, tiles)
@@ -335,8 +362,10 @@ def _partial_args(part: torch.Tensor | None):
 
 
 def _kv_strides(k, v, name):
-    _require(k.stride() == v.stride(), f"{name}: k and v must share strides")
-    return k.stride(0), k.stride(1), k.stride(2)
+    ks = k.stride()
+    if ks != v.stride():
+        raise AssertionError(f"{name}: k and v must share strides")
+    return ks[:3]
 
 
 def bigbird_sparse_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
@@ -395,23 +424,39 @@ def paged_sparse_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.T
     """
     name = "paged_sparse_decode"
     q3 = q.reshape(q.shape[0], q.shape[1], q.shape[-1]) if q.dim() == 4 else q
-    _require(q3.is_cuda and k_pages.is_cuda and v_pages.is_cuda, f"{name} requires GPU tensors")
-    _require(q3.dtype in _DTYPES and k_pages.dtype == q3.dtype and v_pages.dtype == q3.dtype,
-             f"{name}: q/k/v must share an fp16 or bf16 dtype")
-    _require(k_pages.shape == v_pages.shape and k_pages.dim() == 4, f"{name}: pools must be [P, Hkv, page, D]")
-    B, Hq, D = q3.shape
-    _, Hkv, page, Dk = k_pages.shape
-    _require(D == Dk and Hq % Hkv == 0, f"{name}: head mismatch")
-    for t in (block_table, kv_lens, sel, sel_off):
-        _require(t.dtype == torch.int32 and t.device == q3.device, f"{name}: index tensors must be int32 on the GPU")
-    _require(sel.dim() == 3 and sel_off.dim() == 3 and sel_off.shape[2] == 2, f"{name}: bad sel shapes")
-    _require(block_table.dim() == 2 and block_table.size(0) == B,
-             f"{name}: block_table must be [B={B}, max_blocks], got {tuple(block_table.shape)}")
-    _require(kv_lens.shape == (B,), f"{name}: kv_lens must be [B={B}], got {tuple(kv_lens.shape)}")
-    R = sel.shape[1]
-    _require(R in (Hq, Hkv) and sel_off.shape[:2] == (B, R) and sel.shape[0] == B, f"{name}: bad sel rows")
-    _require(sel.stride(2) == 1 and block_table.stride(1) == 1 and kv_lens.is_contiguous()
-             and sel_off.stride(2) == 1, f"{name}: index tensors must be contiguous in the last dim")
+    # One test of everything first: a call that passes formats no message.
+    ok = q3.dim() == 3 and k_pages.dim() == 4 and sel.dim() == 3
+    if ok:
+        B, Hq, D = q3.shape
+        kp_shape = k_pages.shape
+        R, dev = sel.shape[1], q3.device
+        ok = (q3.is_cuda and k_pages.is_cuda and v_pages.is_cuda and q3.dtype in _DTYPES and k_pages.dtype == q3.dtype
+              and v_pages.dtype == q3.dtype and kp_shape == v_pages.shape and D == kp_shape[3] and Hq % kp_shape[1] == 0
+              and block_table.dtype == torch.int32 and kv_lens.dtype == torch.int32 and sel.dtype == torch.int32
+              and sel_off.dtype == torch.int32 and block_table.device == dev and kv_lens.device == dev
+              and sel.device == dev and sel_off.device == dev and sel_off.shape == (B, R, 2) and sel.shape[0] == B
+              and block_table.dim() == 2 and block_table.size(0) == B and kv_lens.shape == (B,)
+              and (R == Hq or R == kp_shape[1]) and sel.stride(2) == 1 and block_table.stride(1) == 1
+              and kv_lens.is_contiguous() and sel_off.stride(2) == 1)
+    if not ok:
+        _require(q3.is_cuda and k_pages.is_cuda and v_pages.is_cuda, f"{name} requires GPU tensors")
+        _require(q3.dtype in _DTYPES and k_pages.dtype == q3.dtype and v_pages.dtype == q3.dtype,
+                 f"{name}: q/k/v must share an fp16 or bf16 dtype")
+        _require(k_pages.shape == v_pages.shape and k_pages.dim() == 4, f"{name}: pools must be [P, Hkv, page, D]")
+        B, Hq, D = q3.shape
+        _, Hkv, page, Dk = k_pages.shape
+        _require(D == Dk and Hq % Hkv == 0, f"{name}: head mismatch")
+        for t in (block_table, kv_lens, sel, sel_off):
+            _require(t.dtype == torch.int32 and t.device == q3.device, f"{name}: index tensors must be int32 on the GPU")
+        _require(sel.dim() == 3 and sel_off.dim() == 3 and sel_off.shape[2] == 2, f"{name}: bad sel shapes")
+        _require(block_table.dim() == 2 and block_table.size(0) == B,
+                 f"{name}: block_table must be [B={B}, max_blocks], got {tuple(block_table.shape)}")
+        _require(kv_lens.shape == (B,), f"{name}: kv_lens must be [B={B}], got {tuple(kv_lens.shape)}")
+        R = sel.shape[1]
+        _require(R in (Hq, Hkv) and sel_off.shape[:2] == (B, R) and sel.shape[0] == B, f"{name}: bad sel rows")
+        _require(sel.stride(2) == 1 and block_table.stride(1) == 1 and kv_lens.is_contiguous()
+                 and sel_off.stride(2) == 1, f"{name}: index tensors must be contiguous in the last dim")
+    Hkv, page = k_pages.size(1), k_pages.size(2)
     if num_splits == 0:
         num_splits = _decode_splits(_decode_units(B, Hq, R), sel.shape[2])
     if out is None:

@@ -121,13 +121,19 @@ def csr_to_block_mask(pairs: torch.Tensor, offsets: torch.Tensor, nkb: int) -> t
     return out
 
 
+def capped_steps(first: int, n: int, cap: int) -> int:
+    """``sum(min(first + i, cap) for i in range(n))`` in closed form (a build asks for it each time)."""
+    ramp = min(max(cap - first, 0), n)       # terms below the cap
+    return ramp * first + ramp * (ramp - 1) // 2 + (n - ramp) * cap
+
+
 def causal_block_keep_ratio(offsets: torch.Tensor, T_q: int, T_k: int, block_size: int) -> float:
     """Kept pairs over the causal block triangle; ``bigbird_pattern.py:108-125``."""
     H = offsets.shape[0]
     nqb = offsets.shape[1] - 1
     nkb = -(-T_k // block_size)
     qbo = max(0, T_k - T_q) // block_size
-    denom = sum(min(qbo + i + 1, nkb) for i in range(nqb))
+    denom = capped_steps(qbo + 1, nqb, nkb)
     if denom <= 0:
         return 0.0
     kept = int(offsets[:, -1].long().sum().item())

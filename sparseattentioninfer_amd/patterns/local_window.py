@@ -11,7 +11,8 @@ from __future__ import annotations
 
 import torch
 
-from sparseattentioninfer_amd.patterns.base import PatternMetadata, SparsePattern, block_mask_to_csr
+from sparseattentioninfer_amd.patterns.base import (PatternMetadata, SparsePattern, block_mask_to_csr,
+                                                    capped_steps)
 from sparseattentioninfer_amd.patterns.bigbird import LazyMaskMetadata
 
 
@@ -73,5 +74,5 @@ class LocalWindowPattern(SparsePattern):
         if T_q == 0 or T_k == 0:
             return 0.0
         qo = max(0, T_k - T_q)
-        kept = sum(min(W, qo + i + 1) for i in range(T_q))
+        kept = capped_steps(qo + 1, T_q, W)
         return min(1.0, kept / (T_q * T_k))

@@ -20,7 +20,7 @@ from collections import OrderedDict
 
 import torch
 
-from .base import PatternMetadata, SparsePattern, block_mask_to_csr
+from .base import PatternMetadata, SparsePattern, block_mask_to_csr, capped_steps
 
 
 def _causal_limit(nqb: int, nkb: int, q_block_offset: int) -> torch.Tensor:
@@ -130,8 +130,14 @@ class _BlockMaskPattern(SparsePattern):
         key = (nqb, nkb, qbo, str(q.device))
         entry = self._cache.get(key)
         if entry is None:
-            pairs, offsets = block_mask_to_csr(self._block_mask(nqb, nkb, qbo, self._device_for(q.device)))
-            kept = int(offsets[:, -1].long().sum())
+            mask = self._block_mask(nqb, nkb, qbo, self._device_for(q.device))
+            if mask.is_cuda:
+                from ..ops import csr_of_mask
+                pairs, offsets, counts = csr_of_mask(mask)
+                kept = sum(counts)
+            else:
+                pairs, offsets = block_mask_to_csr(mask)
+                kept = int(offsets[:, -1].long().sum())
             entry = (pairs.to(q.device), offsets.to(q.device), kept)
             self._cache[key] = entry
             if len(self._cache) > self.CACHE_SIZE:
@@ -139,7 +145,7 @@ class _BlockMaskPattern(SparsePattern):
         else:
             self._cache.move_to_end(key)
         pairs, offsets, kept = entry
-        denom = sum(min(qbo + i + 1, nkb) for i in range(nqb)) * self.rows
+        denom = capped_steps(qbo + 1, nqb, nkb) * self.rows
         kr = min(1.0, kept / denom) if denom > 0 else 0.0
         return PatternMetadata(kind="mask", keep_ratio=kr, block_size=bs,
                                block_pairs=pairs, block_pair_offsets=offsets)
