@@ -138,6 +138,11 @@ int64_t sa_prefill_partial_bytes(int csr_rows, int B, int Hq, int T_q, int T_k, 
 /* Bytes of the optional sa_prefill workspace (counters and the status word). */
 int64_t sa_prefill_workspace_bytes(void);
 
+/* Bytes of a sa_prefill workspace that also holds one work queue per XCD: with
+ * these (8-byte aligned), launches may keep the work of a KV head on one XCD.
+ * Otherwise it is used as a workspace of sa_prefill_workspace_bytes(). */
+int64_t sa_prefill_queue_workspace_bytes(void);
+
 /*
  * Regroups a CSR schedule of block size 16 or 32 -- the granularity of the
  * reference's BigBird layouts, whose CSR block is the next power of two of at

@@ -62,6 +62,7 @@ SIGNATURES = {
     ]),
     "sa_prefill_partial_bytes": (_i64, [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _i64]),
     "sa_prefill_workspace_bytes": (_i64, []),
+    "sa_prefill_queue_workspace_bytes": (_i64, []),
     "sa_block_mask_to_csr": (_i32, [
         _vp, _i64, _i64,
         _i32, _i32, _i32,

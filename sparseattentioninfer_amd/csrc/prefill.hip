@@ -34,7 +34,8 @@
 //  * four-head launches of few query tiles with long lists divide each item's keys over
 //    workgroups, whose fp32 partials a second kernel merges;
 //  * with a workspace, one persistent workgroup per CU slot takes its first work items by its
-//    own index and claims further ones from an atomic counter, heaviest query tiles first.
+//    own index and claims further ones from an atomic counter, heaviest query tiles first --
+//    or, where a KV head's K/V fit an L2, from the counter of its XCD's queue of KV heads.
 //
 // MFMA 32x32x16 lane layouts used (l = lane, g = l / 32):
 //   A (32 x 16): lane l holds row l % 32, k = 8g .. 8g+7
@@ -88,9 +89,9 @@ struct PrefillArgs {
   int tpb_log2;      // log2(block_size / 64): key tiles per CSR block
   int q_offset;
   float scale_log2;  // sm_scale * log2(e)
-  // Persistent mode: the claims word (WS_CLAIMS below) and the status word of the workspace; every
-  // completed launch leaves the claims word zero and the status word as it found it, or with
-  // WS_SKIPPED set.
+  // Persistent mode: the 64-bit words (WS_* below) and the status word of the workspace; every
+  // completed launch leaves the former zero and the status word as it found it, or with WS_SKIPPED
+  // set.
   unsigned long long* claims;
   unsigned int* status;
   // Work-item decoding without integer division: per_tile = R * B * head_splits, and
@@ -113,25 +114,40 @@ struct PrefillArgs {
   int splits;
   uint32_t mul_splits;
   float* part;
+  // Queued launches (queues == N_XCD, otherwise 1): the items in unit order, a unit being what reads
+  // the KV heads of one or a few (b, kvh) -- latest query tiles first, then the unit_heads KV heads, the
+  // per_head items of each -- cut into one contiguous queue per XCD.  per_unit = ntq * per_qt items,
+  // per_qt = unit_heads * per_head, per_head = (R / Hkv) * head_splits.
+  int queues, per_unit, per_qt, per_head, unit_heads, heads_per_kv;
+  uint32_t mul_unit, mul_qt, mul_head, mul_hkv;
   // Timeline launches only (sa_prefill_timeline): TL_WORDS words per workgroup.
   unsigned long long* timeline;
 };
 
-// The persistent-launch workspace: a 64-bit claims word (its low half counts claims, its high half
-// the items that the claiming workgroups have taken so far) and a status word that only the host
-// clears.  A workgroup claims until a claim fails, once; so the claim that reads
-// (claimable items + workgroups - 1) is the launch's last: its workgroup zeroes the word for the next
-// launch, and the high half must then hold every item.  It does not when the word was not zero at
-// launch or launches that overlapped in time shared it: WS_SKIPPED is set, items may have been
-// skipped and their outputs not written, so the caller must not use the output and zeroes the
-// workspace.
-// (Counting finished workgroups instead took two more returning atomics and two device-wide fences
-// of every workgroup, all on one line: 1,024 one-head items of 9 tiles ran 69 us, now 36 us.)
-enum : int { WS_CLAIMS = 0, WS_STATUS = 3, WS_WORDS = 8 };
+// The persistent-launch workspace, in 64-bit words from its first 8-byte boundary: queue x's claims
+// word at 16 x, its finish word at 16 x + 2, the finish word of the queues at 4; and the 32-bit status
+// word (only the host clears it) at byte 12.  Launches with one queue use its claims word only.
+//  * One queue: the claims word's low half counts claims, its high half the items that the claiming
+//    workgroups have taken so far.  A workgroup claims until a claim fails, once; so the claim that
+//    reads (claimable items + workgroups - 1) is the launch's last: its workgroup zeroes the word for
+//    the next launch, and the high half must then hold every item.
+//  * A queue per XCD: a claims word counts the claims made from its queue.  A workgroup whose claim
+//    fails tries one other queue, and has finished when that gives nothing either.  A finish word
+//    counts its queue's owners that have finished (low half) and the items they have taken (high half);
+//    the last owner passes the sum on, and the last queue's zeroes every word; the items must be all.
+// The items are not all when a word was not zero at launch or launches that overlapped in time shared
+// the words: WS_SKIPPED is set, items may have been skipped and their outputs not written, so the
+// caller must not use the output and zeroes the workspace.
+// A workgroup's last claim comes while it still has items to run, so nothing of this is at the end of
+// a launch.  (Two returning atomics on one line and two device-wide fences at the end of every
+// workgroup: 1,024 one-head items of 9 tiles ran 69 us, now 36 us.)
+enum : int { WS_CLAIMS = 0, WS_FINISH = 2, WS_ALL = 4, WS_QUEUE = 16, WS_STATUS = 3, WS_WORDS = 8 };
+constexpr int WS_QUEUE_BYTES = N_XCD * WS_QUEUE * 8;
 constexpr unsigned WS_SKIPPED = 1u;
 
-// A claim of a launch of n_items items, `fixed` of which are dealt by index, by a workgroup that has
-// taken `taken` items since its last one: add_claim's result gives the item, or n_items (none left).
+// One queue: a claim of a launch of n_items items, `fixed` of which are dealt by index, by a workgroup
+// that has taken `taken` items since its last one: add_claim's result gives the item, or n_items (none
+// left).
 __device__ __forceinline__ int claimed_item(unsigned long long* claims, unsigned* status, unsigned long long old,
                                             int taken, int fixed, int n_items) {
   const unsigned n = (unsigned)old;
@@ -797,6 +813,59 @@ struct Prefill {
     return mx * c;  // -inf stays -inf (c > 0)
   }
 
+  // ---- queues (persistent loop) ---------------------------------------------------------------
+  // Queue x holds the items [queue_start(x), queue_start(x + 1)); the workgroups w = x mod queues own
+  // it.  Its first LOOKAHEAD items per owner are dealt, the others claimed, so every item is dealt or
+  // claimed once: an owner leaves its queue only when the queue has run out.
+  enum : int { CL_QUEUE = 0, CL_TAKEN = 1, CL_WORDS = 2 };  // queue claimed from, items taken
+  static __device__ __forceinline__ int queue_start(const PrefillArgs& a, int x, int n_items) {
+    return a.queues == 1 ? x * n_items : (int)((int64_t)n_items * x / N_XCD);
+  }
+  static __device__ __forceinline__ int owners(const PrefillArgs& a) {
+    return a.queues == 1 ? (int)gridDim.x : (int)gridDim.x / N_XCD;
+  }
+
+  // Claim number n of queue x: its item, or n_items where the queue has run out.
+  static __device__ __forceinline__ int queue_item(const PrefillArgs& a, int x, unsigned n, int n_items) {
+    const int s = queue_start(a, x, n_items) + LOOKAHEAD * owners(a);
+    return n < (unsigned)(queue_start(a, x + 1, n_items) - s) ? s + (int)n : n_items;
+  }
+
+  // Thread 0: the item of the claim that read n from the current queue, or n_items (see WS_CLAIMS).
+  // Once a queue has run out, each of its owners looks at one of the other seven, by its index (all of
+  // them looking at all seven counters costs more than it balances, 1,024 workgroups on 8 lines: 8,192
+  // tokens of 32 heads 293 against 280 us, with a window 137 against 124).
+  static __device__ __forceinline__ int queue_claimed(const PrefillArgs& a, int* cl, unsigned n, int n_items) {
+    const int own = (int)blockIdx.x % N_XCD;
+    int x = cl[CL_QUEUE];
+    int v = queue_item(a, x, n, n_items);
+    if (v >= n_items && x == own) {
+      x = (own + 1 + (int)(blockIdx.x / N_XCD) % (N_XCD - 1)) % N_XCD;
+      unsigned long long* c = &a.claims[x * WS_QUEUE + WS_CLAIMS];
+      if (queue_item(a, x, (unsigned)__hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), n_items) < n_items) {
+        v = queue_item(a, x, (unsigned)atomicAdd(c, 1ull), n_items);
+        cl[CL_QUEUE] = x;
+      }
+    }
+    if (v < n_items) {
+      cl[CL_TAKEN] += 1;
+      return v;
+    }
+    unsigned long long taken = (unsigned)cl[CL_TAKEN];
+    unsigned long long old = atomicAdd(&a.claims[own * WS_QUEUE + WS_FINISH], 1ull | (taken << 32));
+    if ((unsigned)old != (unsigned)owners(a) - 1) return n_items;
+    atomicExch(&a.claims[own * WS_QUEUE + WS_FINISH], 0ull);
+    taken += old >> 32;
+    old = atomicAdd(&a.claims[WS_ALL], 1ull | (taken << 32));
+    if ((unsigned)old != N_XCD - 1) return n_items;
+    atomicExch(&a.claims[WS_ALL], 0ull);
+    taken += old >> 32;
+    bool ok = taken == (unsigned long long)n_items;
+    for (int y = 0; y < N_XCD; ++y) ok = (atomicExch(&a.claims[y * WS_QUEUE + WS_CLAIMS], 0ull) >> 32) == 0 && ok;
+    if (!ok) atomicOr(a.status, WS_SKIPPED);
+    return n_items;
+  }
+
   // ---- lookahead metadata (persistent loop) ---------------------------------------------
   // While an item's first tiles load, the persistent loop fetches the CSR row of the next
   // item, the CSR offsets and decoded (qt, r, hs, b) of the item after it and a new claim
@@ -815,6 +884,7 @@ struct Prefill {
     int* vid3;            // id slot of the newly claimed item
     int taken;            // items taken since the last claim; 0: no claim (all items dealt, or none left)
     int fixed;            // items dealt by index
+    int* cl;              // several queues: claim state in LDS (CL_*, thread 0 only)
   };
   static constexpr int RPT = (RC + NT - 1) / NT;  // cached row entries per thread
   struct LookLoads {
@@ -850,7 +920,9 @@ struct Prefill {
         ld.o0 = o[0];
         ld.o1 = o[1];
       }
-      if (lk.taken) ld.nv = add_claim(a.claims, lk.taken);
+      if (lk.taken)
+        ld.nv = a.queues == 1 ? add_claim(a.claims, lk.taken)
+                              : atomicAdd(&a.claims[lk.cl[CL_QUEUE] * WS_QUEUE + WS_CLAIMS], 1ull);
     }
   }
 
@@ -871,7 +943,11 @@ struct Prefill {
       lk.meta2[4] = ld.r2;
       lk.meta2[5] = ld.hs2;
       lk.meta2[6] = ld.b2;
-      lk.vid3[0] = lk.taken ? claimed_item(a.claims, a.status, ld.nv, lk.taken, lk.fixed, lk.n_items) : lk.n_items;
+      int v3 = lk.n_items;
+      if (lk.taken)
+        v3 = a.queues == 1 ? claimed_item(a.claims, a.status, ld.nv, lk.taken, lk.fixed, lk.n_items)
+                           : queue_claimed(a, lk.cl, (unsigned)ld.nv, lk.n_items);
+      lk.vid3[0] = v3;
     }
   }
 
@@ -1486,11 +1562,26 @@ struct Prefill {
   }
 
   // Item index -> (qt, r, hs, b).  Per lane: v may differ between lanes (the startup reads two
-  // items' offsets in two lanes).  Without row_order: query tiles latest first, all rows of a
+  // items' offsets in two lanes).  Queued launches: unit order.  Without row_order: query tiles latest first, all rows of a
   // tile together; with it: row by row (s_row_rank), latest query tiles first within a row.
   static __device__ __forceinline__ void decode_item(const PrefillArgs& a, int v, int& qt, int& r, int& hs, int& b) {
     uint32_t rem;
     if constexpr (KS) v = (int)fast_div((uint32_t)v, (uint32_t)a.splits, a.mul_splits);
+    if (a.queues > 1) {  // unit order
+      const uint32_t u = fast_div((uint32_t)v, (uint32_t)a.per_unit, a.mul_unit);
+      const uint32_t ru = (uint32_t)v - u * (uint32_t)a.per_unit;
+      const uint32_t t = fast_div(ru, (uint32_t)a.per_qt, a.mul_qt);
+      qt = a.ntq - 1 - (int)t;
+      const uint32_t w = ru - t * (uint32_t)a.per_qt;
+      const uint32_t uh = fast_div(w, (uint32_t)a.per_head, a.mul_head);
+      const uint32_t rh = w - uh * (uint32_t)a.per_head;
+      const uint32_t rr = fast_div(rh, (uint32_t)a.head_splits, a.mul_hs);
+      hs = (int)(rh - rr * (uint32_t)a.head_splits);
+      const uint32_t head = u * (uint32_t)a.unit_heads + uh;  // b Hkv + kvh
+      b = (int)fast_div(head, (uint32_t)a.Hkv, a.mul_hkv);
+      r = ((int)head - b * a.Hkv) * (a.R == a.Hkv ? 1 : a.heads_per_kv) + (int)rr;
+      return;
+    }
     if (a.row_order && v >= a.head_items) {
       const uint32_t w = (uint32_t)(v - a.head_items);
       const uint32_t k = fast_div(w, (uint32_t)a.per_group, a.mul_group);
@@ -1576,12 +1667,17 @@ struct Prefill {
     // top reads an item's whole slot (and the ids and offsets of the next two) in one batch.
     __shared__ __attribute__((aligned(16))) int s_meta[4][8];
     const int tid = threadIdx.x;
+    __shared__ int s_cl[CL_WORDS];
     if (tid == 0) {
-      const int g = (int)gridDim.x, w = (int)blockIdx.x;
-      const bool many = n_items > LOOKAHEAD * g;
-      s_meta[0][0] = many ? LOOKAHEAD * w : w;
-      s_meta[1][0] = many ? LOOKAHEAD * w + 1 : 2 * g - 1 - w;
-      s_meta[2][0] = many ? LOOKAHEAD * w + 2 : 2 * g + w;
+      const int x = a.queues == 1 ? 0 : (int)blockIdx.x % N_XCD, g = owners(a);
+      const int w = a.queues == 1 ? (int)blockIdx.x : (int)blockIdx.x / N_XCD;
+      const bool many = n_items > LOOKAHEAD * (int)gridDim.x;  // always with queues
+      const int s = queue_start(a, x, n_items);
+      s_meta[0][0] = s + (many ? LOOKAHEAD * w : w);
+      s_meta[1][0] = s + (many ? LOOKAHEAD * w + 1 : 2 * g - 1 - w);
+      s_meta[2][0] = s + (many ? LOOKAHEAD * w + 2 : 2 * g + w);
+      s_cl[CL_QUEUE] = x;
+      s_cl[CL_TAKEN] = LOOKAHEAD;
     }
     __syncthreads();
     if (tid < 2) {
@@ -1641,6 +1737,7 @@ struct Prefill {
       lk.fixed = LOOKAHEAD * (int)gridDim.x;
       // the first claim counts the dealt items, a later one the item of the claim before it
       lk.taken = n_items <= lk.fixed || lk.v2 >= n_items ? 0 : i == 0 ? LOOKAHEAD : 1;
+      lk.cl = s_cl;
       const int qt = __builtin_amdgcn_readfirstlane(m0.w);
       const int r = __builtin_amdgcn_readfirstlane(m0b.x);
       const int hs = __builtin_amdgcn_readfirstlane(m0b.y);
@@ -1766,9 +1863,12 @@ static int num_cus() {
 }
 
 template <bool BF16, int D, int HW, int NS, bool SUB>
-static hipError_t launch_sub(const PrefillArgs& a, int64_t n_items, int64_t item_grid, hipStream_t s) {
+static hipError_t launch_sub(PrefillArgs a, int64_t n_items, int64_t item_grid, hipStream_t s) {
   int64_t grid = item_grid;
   if (a.claims) grid = std::min<int64_t>(n_items, (int64_t)num_cus() * resident_per_cu<BF16, D, HW, NS, SUB>());
+  // Queues need claims, owners in equal numbers and LOOKAHEAD items for each.
+  if (n_items <= LOOKAHEAD * grid || grid % N_XCD) a.queues = 1;
+  if (a.queues > 1) a.row_order = 0;
   hipLaunchKernelGGL((prefill_kernel<BF16, D, HW, NS, SUB>), dim3(grid), dim3(128 * HW * NS), 0, s, a);
   return hipGetLastError();
 }
@@ -1981,14 +2081,38 @@ static int prefill_impl(const char* fn, int dtype,
     return set_error(SA_E_ALIGN, "%s: workspace must be 4-byte aligned", fn);
   a.claims = nullptr;
   a.status = nullptr;
-  if (workspace) {  // the claims word at the first 8-byte boundary of the 4-byte aligned workspace
+  if (workspace) {  // 64-bit words from the first 8-byte boundary of the 4-byte aligned workspace
     auto* w = static_cast<unsigned int*>(workspace);
-    a.claims = reinterpret_cast<unsigned long long*>(w + WS_CLAIMS + ((reinterpret_cast<uintptr_t>(w) >> 2) & 1));
+    a.claims = reinterpret_cast<unsigned long long*>(w + ((reinterpret_cast<uintptr_t>(w) >> 2) & 1));
     a.status = w + WS_STATUS;
   }
 
   const int64_t per_tile = (int64_t)a.R * B * a.head_splits;
   const int64_t n_items = (int64_t)a.ntq * per_tile;
+  // Queues: one XCD keeps to a few KV heads, whose K/V its L2 can hold (past the L2s the Infinity Cache
+  // serves 26-30 B/ns per CU, an L2 117-145).  Items that read a whole KV head's rows one head at a time
+  // gain most: 8,192 tokens of 32 heads, blocks of 32, 335 us with one queue, 280 with eight; a window of
+  // 512 175 / 124 us; 32,768 tokens 528 / 449; rows whose lengths differ by a group's budget (2 to 30 %)
+  // 396 / 358.  Four heads to an item read less: dense 8,192 tokens 716 / 604, blocks drawn from 8,192
+  // tokens 319 / 315, and past the L2 nothing: the 32K-token prompt (16 MB per head, groups of different
+  // densities) 335 / 392 us.
+  const int64_t heads = (int64_t)B * Hkv, head_bytes = (int64_t)T_k * D * 4;
+  constexpr int64_t L2_BYTES = 4 << 20;
+  a.queues = 1;
+  if (workspace && workspace_bytes >= WS_QUEUE_BYTES && (reinterpret_cast<uintptr_t>(workspace) & 7) == 0 && !timeline &&
+      a.splits == 1 && heads % N_XCD == 0 && (hw < 4 || head_bytes <= L2_BYTES))
+    a.queues = N_XCD;
+  a.unit_heads = 1;  // the largest divisor of a queue's heads that fits
+  for (int64_t g = 2; g <= heads / N_XCD && g * head_bytes <= L2_BYTES; ++g)
+    if ((heads / N_XCD) % g == 0) a.unit_heads = (int)g;
+  a.heads_per_kv = Hq / Hkv;
+  a.per_head = (csr_rows == Hkv ? 1 : a.heads_per_kv) * a.head_splits;
+  a.per_qt = a.unit_heads * a.per_head;
+  a.per_unit = a.ntq * a.per_qt;
+  a.mul_unit = div_mul((uint32_t)a.per_unit);
+  a.mul_qt = div_mul((uint32_t)a.per_qt);
+  a.mul_head = div_mul((uint32_t)a.per_head);
+  a.mul_hkv = div_mul((uint32_t)Hkv);
   const int64_t chunk = XCD_CHUNK * per_tile;
   const int64_t item_grid = ceil_div(ceil_div(n_items, chunk), N_XCD) * N_XCD * chunk;
   if (item_grid > 0x7fffffff) return set_error(SA_E_SHAPE, "%s: %lld work items is too many", fn, (long long)n_items);
@@ -2100,3 +2224,5 @@ extern "C" int64_t sa_prefill_timeline_words(int dtype) {
 }
 
 extern "C" int64_t sa_prefill_workspace_bytes(void) { return sa::WS_WORDS * (int64_t)sizeof(unsigned int); }
+
+extern "C" int64_t sa_prefill_queue_workspace_bytes(void) { return sa::WS_QUEUE_BYTES; }

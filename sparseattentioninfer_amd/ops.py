@@ -47,7 +47,7 @@ def _prefill_workspace(t: torch.Tensor) -> torch.Tensor:
     key = (t.device.index, stream)
     ws = _PREFILL_WS.get(key)
     if ws is None:
-        nbytes = int(_lib.load().sa_prefill_workspace_bytes())
+        nbytes = int(_lib.load().sa_prefill_queue_workspace_bytes())
         ws = torch.zeros((nbytes + 3) // 4, dtype=torch.int32, device=t.device)
         _PREFILL_WS[key] = ws
     return ws
