@@ -302,11 +302,12 @@ def universal_sparse_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if T_q == 1 and q_offset == T_k - 1:
         if nqb != 1:
             raise AssertionError(f"{name}: decode expects one CSR query block, got {nqb}")
-        # Lists of 1,024 keys and more are split over workgroups: unsplit, a row's list is read by one CU
-        # (4 sequences of 8,191 tokens, 32 heads, 8 KV heads: 137 us; split by 8, 27 us).  Shorter ones are
-        # not: the partials and the combine cost an eager call 5 us of launching (256 keys of 8 heads: 15 us
-        # unsplit, 20 us split by 8).
-        splits = _decode_splits(_decode_units(B, Hq, R), pairs.size(1)) if pairs.size(1) * block_size >= 1024 else 1
+        # Lists of 512 KB and more (K and V of 1,024 keys of 128) are split over workgroups: unsplit, a row's
+        # list is read by one CU at about 30 B/ns (4 sequences of 8,191 tokens, 32 heads, 8 KV heads: 137 us;
+        # split by 8, 27 us).  Shorter ones are not: the partials and the combine cost an eager call 5 us of
+        # launching (256 keys of 8 heads: 15 us unsplit, 20 us split by 8; 1,792 keys of 64 15.5 and 16.7).
+        long = pairs.size(1) * block_size * D >= 1024 * 128
+        splits = decode_splits(B, Hq, R, pairs.size(1)) if long else 1
         ws_bytes = splits * B * Hq * (D + 2) * 4 if splits > 1 else 0
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
         status = lib.sa_decode(
@@ -388,23 +389,20 @@ def auto_decode_splits(B: int, rows: int, max_sel: int, target_workgroups: int =
     return max(1, min(want, max_sel // 2, 16))
 
 
-def _decode_splits(units: int, max_sel: int) -> int:
-    """Splits of each block list for one decode launch of ``units`` workgroups unsplit: up to one
-    workgroup per CU (256), at least two blocks per split, at most 32 splits.
+def decode_splits(B: int, Hq: int, rows: int, max_sel: int) -> int:
+    """Splits of each block list for one decode launch: up to one workgroup per CU (256), at least two
+    blocks per split, at most 32 splits.
 
-    A workgroup's four waves keep about 64 KB of loads in flight, so 256 of them already draw HBM's
-    rate and further splits only add to the combine.  Measured (us): 4 sequences of 8,191 tokens (32
-    units, 134 MB) 41.7 / 27.1 / 28.5 / 34.2 with 4 / 8 / 16 / 32 splits; one of 32,000 (8 units) 72.9 /
-    42.0 / 28.8 / 31.9 with 8 / 16 / 32 / 64; 14 blocks of 64 kept by 64 units 19.5 / 15.3 / 13.3 / 13.2
-    with 1 / 2 / 4 / 8, by 128 units 20.1 / 17.6 / 19.0 with 1 / 2 / 4, by 192 units 22.0 / 25.2 with 1 / 2.
+    An unsplit launch has one workgroup per sequence, row and up to four of the row's query heads.  A
+    workgroup's four waves keep about 64 KB of loads in flight, so 256 of them already draw HBM's rate
+    and further splits only add to the combine.  Measured (us): 4 sequences of 8,191 tokens (32
+    workgroups unsplit, 134 MB) 41.7 / 27.1 / 28.5 / 34.2 with 4 / 8 / 16 / 32 splits; one of 32,000 (8)
+    72.9 / 42.0 / 28.8 / 31.9 with 8 / 16 / 32 / 64; 14 blocks of 64 kept by 64 workgroups 19.5 / 15.3 /
+    13.3 / 13.2 with 1 / 2 / 4 / 8, by 128 20.1 / 17.6 / 19.0 with 1 / 2 / 4, by 192 22.0 / 25.2 with 1 / 2.
     """
-    return max(1, min(256 // max(1, units), max_sel // 2, 32))
-
-
-def _decode_units(B: int, Hq: int, rows: int) -> int:
-    """Workgroups of an unsplit decode launch: up to four query heads of a row share one."""
     per_row = Hq // rows
-    return B * rows * (per_row // 4 if per_row % 4 == 0 else per_row // 2 if per_row % 2 == 0 else per_row)
+    units = B * rows * (per_row // 4 if per_row % 4 == 0 else per_row // 2 if per_row % 2 == 0 else per_row)
+    return max(1, min(256 // max(1, units), max_sel // 2, 32))
 
 
 def paged_sparse_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
@@ -458,7 +456,7 @@ def paged_sparse_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.T
                  and sel_off.stride(2) == 1, f"{name}: index tensors must be contiguous in the last dim")
     Hkv, page = k_pages.size(1), k_pages.size(2)
     if num_splits == 0:
-        num_splits = _decode_splits(_decode_units(B, Hq, R), sel.shape[2])
+        num_splits = decode_splits(B, Hq, R, sel.shape[2])
     if out is None:
         out = torch.empty(B, Hq, D, dtype=q3.dtype, device=q3.device)
     lib = _lib.load()

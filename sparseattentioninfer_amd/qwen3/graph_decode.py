@@ -114,7 +114,7 @@ class _LayerSchedule:
         self.row_of = row_of
         self.sel = self.sel_off = None  # views of the decoder's gathered selections (set by the decoder)
         self.rows = R
-        self.num_splits = ops.auto_decode_splits(batch, R, self.width)
+        self.num_splits = ops.decode_splits(batch, H, R, self.width)   # as the eager paged decode picks it
         need = ops.decode_workspace_bytes(batch, H, D, self.num_splits)
         self.workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=device)
 

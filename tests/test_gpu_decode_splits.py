@@ -1,5 +1,5 @@
 """Contiguous decode (``universal_sparse_attn`` with one query) around the list lengths from which a
-block list is split over workgroups: just below and at 1,024 keys, lists of a few blocks more than the
+block list is split over workgroups: just below and at 512 KB of K and V, lists of a few blocks more than the
 splits, the 32-split cap, ragged last blocks; and the paged entry point's own choice (``num_splits=0``)."""
 import sys
 
@@ -17,7 +17,7 @@ DEV = "cuda"
 
 @pytest.mark.parametrize("B,Hq,Hkv,rows,D,bs,T", [
     (1, 8, 2, 2, 128, 64, 959), (1, 8, 2, 2, 128, 64, 961), (1, 8, 2, 8, 128, 64, 1025), (2, 6, 3, 3, 64, 16, 1024),
-    (1, 4, 1, 1, 128, 64, 4480), (1, 4, 1, 1, 64, 128, 9000), (3, 16, 2, 2, 128, 32, 2051), (40, 8, 8, 8, 64, 64, 1500)])
+    (1, 4, 1, 1, 128, 64, 4480), (1, 4, 1, 1, 64, 128, 9000), (3, 16, 2, 2, 128, 32, 2051), (40, 8, 8, 8, 64, 64, 1500), (1, 4, 1, 1, 64, 64, 2048)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_split_decode_matches_the_oracle(B, Hq, Hkv, rows, D, bs, T, dtype):
     print(f"[decode splits] B={B} heads={Hq}/{Hkv} rows={rows} D={D} bs={bs} T={T} {dtype}", flush=True)
