@@ -429,15 +429,25 @@ __device__ __forceinline__ uint32_t sl_lds(const void* p) {
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)(p);
 }
 
-// 16 bytes per lane from a per-lane address into LDS at M0 + 16 lane.
+// 16 bytes per lane from a per-lane address into LDS at M0 + 16 lane; NT: non-temporal.
+template <bool NT>
 __device__ __forceinline__ void sl_load16(const void* vaddr, uint32_t lds) {
-  asm volatile(
-      "s_mov_b32 m0, %1\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, off"
-      :
-      : "v"(vaddr), "s"(lds)
-      : "memory", "m0");
+  if constexpr (NT)
+    asm volatile(
+        "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %0, off nt"
+        :
+        : "v"(vaddr), "s"(lds)
+        : "memory", "m0");
+  else
+    asm volatile(
+        "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %0, off"
+        :
+        : "v"(vaddr), "s"(lds)
+        : "memory", "m0");
 }
 
 // NWV waves, 16 output columns each.  A stage holds the workgroup's 16 NWV W rows and the 8 x
@@ -445,7 +455,8 @@ __device__ __forceinline__ void sl_load16(const void* vaddr, uint32_t lds) {
 // ACT: W's rows are Qwen3MLP's gate and up rows interleaved (row 2i = gate i, row 2i + 1 = up i)
 // and out[m, i] = SwiGLU of the pair, rounded as sa_gemm_skinny then sa_swiglu round it (the
 // pair sits in adjacent lanes of one wave).
-template <bool BF16, int NWV, bool ACT>
+// NT: W is read non-temporally (sl_nt).
+template <bool BF16, int NWV, bool ACT, bool NT>
 __global__ __launch_bounds__(64 * NWV) void skinny_lds_kernel(const elem_t* x, int64_t x_st, const elem_t* w,
                                                               int64_t w_st, elem_t* out, int64_t out_st, int M,
                                                               int N, int K) {
@@ -478,10 +489,10 @@ __global__ __launch_bounds__(64 * NWV) void skinny_lds_kernel(const elem_t* x, i
     const uint32_t b = base + (st % SL_NS) * SB;
     const int k0 = st * SL_KC;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) sl_load16(wsrc[i] + k0, b + 1024 * (4 * wave + i));
+    for (int i = 0; i < 4; ++i) sl_load16<NT>(wsrc[i] + k0, b + 1024 * (4 * wave + i));
 #pragma unroll
     for (int j = 0; j < XI; ++j)
-      if (XR >= 4 || lane < XR * 16) sl_load16(xsrc[j] + k0, b + WB + 256 * XR * wave + 1024 * j);
+      if (XR >= 4 || lane < XR * 16) sl_load16<false>(xsrc[j] + k0, b + WB + 256 * XR * wave + 1024 * j);
   };
   // Operand offsets within a stage: B = W row 16 wave + lane % 16, A = x row (lane % 16) & 7;
   // k-chunk 4 ks + lane / 16.
@@ -533,8 +544,26 @@ __global__ __launch_bounds__(64 * NWV) void skinny_lds_kernel(const elem_t* x, i
 }
 
 // Two waves (32 columns) per workgroup: measured best against one and four at the Qwen3-4B decode
-// shapes with the weights streamed from HBM (q|k|v 8.0 us, gate|up 21 us, LM head 134 us).
+// shapes with the weights streamed from HBM (q|k|v 8.0 us, gate|up 21 us, LM head 134 us, all read temporally).
 constexpr int SL_NWV = 2;
+
+// W of 64 MB and more is read non-temporally: one pass over it fills the caches with lines that nothing
+// reads again.  The feed-forward half and output head of a 2560 x 9728 layer with 151,936 tokens, 8 rows
+// (gate|up 100 MB, LM head 778 MB): 185.3 -> 165.2 us, 5.0 -> 5.6 TB/s.  Smaller weights may still be in
+// the Infinity Cache when a step returns to them: with q|k|v (31 MB) and o (21 MB) read non-temporally an
+// attention half took 56.3 us, without 55.7; and the down product (50 MB, dot products) gained nothing
+// (165.8 with, 165.2 without).
+static bool sl_nt(int64_t N, int64_t K) { return N * K * 2 >= (int64_t)64 << 20; }
+
+template <bool BF16, bool ACT>
+static void launch_skinny_lds(const elem_t* x, int64_t x_st, const elem_t* w, int64_t w_st, elem_t* out,
+                              int64_t out_st, int M, int N, int K, hipStream_t s) {
+  const dim3 g((N + 16 * SL_NWV - 1) / (16 * SL_NWV)), b(64 * SL_NWV);
+  if (sl_nt(N, K))
+    hipLaunchKernelGGL((skinny_lds_kernel<BF16, SL_NWV, ACT, true>), g, b, 0, s, x, x_st, w, w_st, out, out_st, M, N, K);
+  else
+    hipLaunchKernelGGL((skinny_lds_kernel<BF16, SL_NWV, ACT, false>), g, b, 0, s, x, x_st, w, w_st, out, out_st, M, N, K);
+}
 
 // Dot-product kernel: rows per batch and workgroups per CU, measured at the Qwen3-4B decode shapes
 // with the weights streamed from HBM: wide products (N >= 64 per CU: gate|up, LM head) take 4 rows per batch and
@@ -547,8 +576,7 @@ static void launch_skinny(const elem_t* x, int64_t x_st, const elem_t* w, int64_
   // (q|k|v, gate|up and the LM head of Qwen3-4B: 20-30 % faster); narrower ones (o, down: 80
   // column tiles) keep more workgroups busy on the dot-product kernel.
   if (K % SL_KC == 0 && N >= 24 * num_cus_layer()) {
-    hipLaunchKernelGGL((skinny_lds_kernel<BF16, SL_NWV, false>), dim3((N + 16 * SL_NWV - 1) / (16 * SL_NWV)),
-                       dim3(64 * SL_NWV), 0, s, x, x_st, w, w_st, out, out_st, M, N, K);
+    launch_skinny_lds<BF16, false>(x, x_st, w, w_st, out, out_st, M, N, K, s);
     return;
   }
   if (N >= 64 * num_cus_layer())
@@ -601,16 +629,13 @@ extern "C" int sa_gemm_skinny_swiglu(int dtype, const void* x, int64_t x_stride,
     return set_error(SA_E_ALIGN, "sa_gemm_skinny_swiglu: x and W rows must be 16-byte aligned");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int N = 2 * I;
-  const dim3 g((N + 16 * SL_NWV - 1) / (16 * SL_NWV)), b(64 * SL_NWV);
   auto xe = static_cast<const elem_t*>(x);
   auto we = static_cast<const elem_t*>(w_gate_up);
   auto oe = static_cast<elem_t*>(out);
   if (dtype == SA_DTYPE_BF16)
-    hipLaunchKernelGGL((skinny_lds_kernel<true, SL_NWV, true>), g, b, 0, s, xe, x_stride, we, w_stride, oe,
-                       out_stride, M, N, K);
+    launch_skinny_lds<true, true>(xe, x_stride, we, w_stride, oe, out_stride, M, N, K, s);
   else
-    hipLaunchKernelGGL((skinny_lds_kernel<false, SL_NWV, true>), g, b, 0, s, xe, x_stride, we, w_stride, oe,
-                       out_stride, M, N, K);
+    launch_skinny_lds<false, true>(xe, x_stride, we, w_stride, oe, out_stride, M, N, K, s);
   const hipError_t err = hipGetLastError();
   return err == hipSuccess ? 0
                            : set_error((int)err, "sa_gemm_skinny_swiglu: launch failed: %s", hipGetErrorString(err));
