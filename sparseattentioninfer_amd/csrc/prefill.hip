@@ -1646,14 +1646,14 @@ struct Prefill {
       item<false>(a, qt, r, hs, b, sKV, s_ml, s_row, s_mask, nullptr);
   }
 
-  // Persistent loop with lookahead.  The first LOOKAHEAD items of a workgroup w are fixed
-  // by w, later ones are claimed from the counter.  (Claimed ahead, the first ones all went to the
-  // workgroups that started first, three each: 128 items of 64-79 tiles -- 1,000 queries of 32
-  // heads on 5,000 keys -- ran on 43 CUs, 297 us; one item per workgroup takes 107 us.)  With fewer
-  // items than LOOKAHEAD per workgroup, item w comes first and the second round runs in reverse, so
-  // the workgroup with the lightest first item takes the heaviest second one; with more, w takes
-  // three neighbouring items as a claim would have given it (w, 2g - 1 - w, 2g + w there: prefill of
-  // 32K tokens 332.7 against 330.0 us).
+  // Persistent loop with lookahead.  The first LOOKAHEAD items of a workgroup w (of g) are fixed by w:
+  // w, 2g - 1 - w and 2g + w, so that the workgroup with the lightest first item takes the heaviest
+  // second one; later ones are claimed from the counter.  (Claimed ahead, the first ones all went to the
+  // workgroups that started first, three each: 128 items of 64-79 tiles -- 1,000 queries of 32 heads on
+  // 5,000 keys -- ran on 43 CUs, 297 us; one item per workgroup takes 107 us.  Three neighbours, 3w to
+  // 3w + 2, give a few workgroups the longest three: four items per workgroup, dense 8,192 tokens of 32
+  // heads 711 us against 581; one dense KV head among eight of five blocks 498 against 208; six per
+  // workgroup, dense 12,288 tokens 1,266 against 1,218; the 32K-token prompt, 16 per workgroup, the same.)
   // Item i of this workgroup finds in LDS its id,
   // CSR offsets and (qt, r, hs, b) (slot i % 4 of s_meta) and its row (row cache i % 2), and
   // the id, offsets and row of item i + 1 and the id of item i + 2; its prologue fetches the
@@ -1671,11 +1671,10 @@ struct Prefill {
     if (tid == 0) {
       const int x = a.queues == 1 ? 0 : (int)blockIdx.x % N_XCD, g = owners(a);
       const int w = a.queues == 1 ? (int)blockIdx.x : (int)blockIdx.x / N_XCD;
-      const bool many = n_items > LOOKAHEAD * (int)gridDim.x;  // always with queues
       const int s = queue_start(a, x, n_items);
-      s_meta[0][0] = s + (many ? LOOKAHEAD * w : w);
-      s_meta[1][0] = s + (many ? LOOKAHEAD * w + 1 : 2 * g - 1 - w);
-      s_meta[2][0] = s + (many ? LOOKAHEAD * w + 2 : 2 * g + w);
+      s_meta[0][0] = s + w;
+      s_meta[1][0] = s + 2 * g - 1 - w;
+      s_meta[2][0] = s + 2 * g + w;
       s_cl[CL_QUEUE] = x;
       s_cl[CL_TAKEN] = LOOKAHEAD;
     }
