@@ -114,7 +114,7 @@ struct PrefillArgs {
   int splits;
   uint32_t mul_splits;
   float* part;
-  // Queued launches (queues == N_XCD, otherwise 1): the items in unit order, a unit being what reads
+  // Launches with queues (queues == N_XCD, otherwise 1), if their rows are even: the items in unit order, a unit being what reads
   // the KV heads of one or a few (b, kvh) -- latest query tiles first, then the unit_heads KV heads, the
   // per_head items of each -- cut into one contiguous queue per XCD.  per_unit = ntq * per_qt items,
   // per_qt = unit_heads * per_head, per_head = (R / Hkv) * head_splits.
@@ -165,6 +165,9 @@ __device__ __forceinline__ unsigned long long add_claim(unsigned long long* clai
 // CSR rows of a persistent launch in descending order of retained blocks (row_order).
 constexpr int MAX_ORDERED_ROWS = 256;
 __shared__ int s_row_rank[MAX_ORDERED_ROWS];
+
+// Whether a launch with queues (PrefillArgs::queues) uses them: if its rows are even (rows_even).
+__shared__ int s_queued;
 
 // Timeline instantiation (TL) of the persistent four-head loop: shader-clock cycles (s_memtime)
 // spent in each phase of an item, summed over the workgroup's items, for the first wave of each
@@ -818,11 +821,37 @@ struct Prefill {
   // it.  Its first LOOKAHEAD items per owner are dealt, the others claimed, so every item is dealt or
   // claimed once: an owner leaves its queue only when the queue has run out.
   enum : int { CL_QUEUE = 0, CL_TAKEN = 1, CL_WORDS = 2 };  // queue claimed from, items taken
+  static __device__ __forceinline__ bool queued(const PrefillArgs& a) { return !KS && a.queues > 1 && s_queued; }
   static __device__ __forceinline__ int queue_start(const PrefillArgs& a, int x, int n_items) {
-    return a.queues == 1 ? x * n_items : (int)((int64_t)n_items * x / N_XCD);
+    return queued(a) ? (int)((int64_t)n_items * x / N_XCD) : x * n_items;
   }
   static __device__ __forceinline__ int owners(const PrefillArgs& a) {
-    return a.queues == 1 ? (int)gridDim.x : (int)gridDim.x / N_XCD;
+    return queued(a) ? (int)gridDim.x / N_XCD : (int)gridDim.x;
+  }
+
+  // Whether no CSR row holds much more than its share of the schedule's blocks.  Every wave finds out
+  // for itself, from the same reads.  Only then may the place of an item say who runs it: on one XCD a
+  // heavy KV head has an eighth of the chip, and a workgroup that holds three items cannot give the
+  // other two away while it runs a long one.  Longest row over the mean row (r) against the time (us).
+  // Four heads to an item, one queue / a queue per XCD: 8,192 tokens of 32 heads, r = 1.04 173 / 173, 1.08
+  // 172 / 174, 1.12 169 / 171; 16,384 tokens, head dim 64, 1.04 221 / 218, 1.08 217 / 221, 1.12 215 / 226;
+  // one dense KV head of eight, r = 5.2, 212 / 405.  One head to an item, 8,192 tokens of 32 heads, every
+  // item claimed when the last has ended / three dealt and a queue per XCD: r = 1.2 216 / 200, 1.4 218 / 220,
+  // 1.7 223 / 270, 5.2 274 / 545.
+  static __device__ __forceinline__ bool rows_even(const PrefillArgs& a) {
+    float sum = 0.f, longest = 0.f;
+    for (int r = threadIdx.x & 63; r < a.R; r += 64) {
+      const int32_t* o = a.offsets + r * a.offsets_stride;
+      const float len = (float)(o[a.nqb] - o[0]);
+      sum += len;
+      longest = fmaxf(longest, len);
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+      sum += __shfl_xor(sum, d);
+      longest = fmaxf(longest, __shfl_xor(longest, d));
+    }
+    return longest * (float)a.R <= sum * (PIPE ? 1.0625f : 1.25f);
   }
 
   // Claim number n of queue x: its item, or n_items where the queue has run out.
@@ -921,8 +950,8 @@ struct Prefill {
         ld.o1 = o[1];
       }
       if (lk.taken)
-        ld.nv = a.queues == 1 ? add_claim(a.claims, lk.taken)
-                              : atomicAdd(&a.claims[lk.cl[CL_QUEUE] * WS_QUEUE + WS_CLAIMS], 1ull);
+        ld.nv = queued(a) ? atomicAdd(&a.claims[lk.cl[CL_QUEUE] * WS_QUEUE + WS_CLAIMS], 1ull)
+                          : add_claim(a.claims, lk.taken);
     }
   }
 
@@ -945,8 +974,8 @@ struct Prefill {
       lk.meta2[6] = ld.b2;
       int v3 = lk.n_items;
       if (lk.taken)
-        v3 = a.queues == 1 ? claimed_item(a.claims, a.status, ld.nv, lk.taken, lk.fixed, lk.n_items)
-                           : queue_claimed(a, lk.cl, (unsigned)ld.nv, lk.n_items);
+        v3 = queued(a) ? queue_claimed(a, lk.cl, (unsigned)ld.nv, lk.n_items)
+                       : claimed_item(a.claims, a.status, ld.nv, lk.taken, lk.fixed, lk.n_items);
       lk.vid3[0] = v3;
     }
   }
@@ -1567,7 +1596,7 @@ struct Prefill {
   static __device__ __forceinline__ void decode_item(const PrefillArgs& a, int v, int& qt, int& r, int& hs, int& b) {
     uint32_t rem;
     if constexpr (KS) v = (int)fast_div((uint32_t)v, (uint32_t)a.splits, a.mul_splits);
-    if (a.queues > 1) {  // unit order
+    if (queued(a)) {  // unit order
       const uint32_t u = fast_div((uint32_t)v, (uint32_t)a.per_unit, a.mul_unit);
       const uint32_t ru = (uint32_t)v - u * (uint32_t)a.per_unit;
       const uint32_t t = fast_div(ru, (uint32_t)a.per_qt, a.mul_qt);
@@ -1658,8 +1687,8 @@ struct Prefill {
   // CSR offsets and (qt, r, hs, b) (slot i % 4 of s_meta) and its row (row cache i % 2), and
   // the id, offsets and row of item i + 1 and the id of item i + 2; its prologue fetches the
   // row of item i + 1, the offsets and (qt, r, hs, b) of item i + 2 and claims item i + 3
-  // (Look).  Claims only grow, so the first id past the end ends the loop in every wave at
-  // once.
+  // (Look).  The ids after one past the end are past it too, so the first such id ends the loop, in
+  // every wave at once.
   static __device__ __forceinline__ void run_lookahead(const PrefillArgs& a, int n_items, char* sKV, char* sQ,
                                                        float* s_ml, int32_t* s_row, int32_t* s_mask) {
     int vb_first = 0;  // V buffer free for the next item's first tile
@@ -1669,8 +1698,8 @@ struct Prefill {
     const int tid = threadIdx.x;
     __shared__ int s_cl[CL_WORDS];
     if (tid == 0) {
-      const int x = a.queues == 1 ? 0 : (int)blockIdx.x % N_XCD, g = owners(a);
-      const int w = a.queues == 1 ? (int)blockIdx.x : (int)blockIdx.x / N_XCD;
+      const int x = queued(a) ? (int)blockIdx.x % N_XCD : 0, g = owners(a);
+      const int w = queued(a) ? (int)blockIdx.x / N_XCD : (int)blockIdx.x;
       const int s = queue_start(a, x, n_items);
       s_meta[0][0] = s + w;
       s_meta[1][0] = s + 2 * g - 1 - w;
@@ -1750,6 +1779,21 @@ struct Prefill {
     }
   }
 
+  // Persistent loop of one- and two-head workgroups over uneven rows: one queue, and every item is
+  // claimed when the one before it has ended.
+  static __device__ __forceinline__ void run_claims(const PrefillArgs& a, int n_items, char* sKV, char* sQ, float* s_ml,
+                                                    int32_t* s_row, int32_t* s_mask) {
+    __shared__ int s_item;
+    for (int taken = 0;; taken = 1) {
+      if (threadIdx.x == 0) s_item = claimed_item(a.claims, a.status, add_claim(a.claims, taken), taken, 0, n_items);
+      __syncthreads();
+      const int v = s_item;
+      __syncthreads();
+      if (v >= n_items) break;
+      process(a, v, sKV, sQ, s_ml, s_row, s_mask);
+    }
+  }
+
   static __device__ void run(const PrefillArgs& a) {
     __shared__ __attribute__((aligned(16))) char sKV[LDS_KV];
     __shared__ __attribute__((aligned(16))) char sQ[LDS_Q];
@@ -1786,7 +1830,19 @@ struct Prefill {
       const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
       if (wave % HW == 0 && (threadIdx.x & 63) == 0) s_tl[wave / HW][TL_NOW] = (unsigned)__builtin_amdgcn_s_memtime();
     }
-    if (a.row_order) rank_rows(a, reinterpret_cast<int*>(sKV));  // K/V buffers are free here
+    // Up to two items per workgroup the second round, which runs in reverse, balances uneven rows as well
+    // as claims do (4,096 tokens of 16 heads, one dense KV head of eight: 118 us dealt, 112 claimed; equal
+    // windows 38 against 44).
+    const bool even = a.queues > 1 || (!PIPE && n_items > 2 * (int)gridDim.x) ? rows_even(a) : true;
+    if (threadIdx.x == 0) s_queued = even;
+    if (a.row_order && !(even && a.queues > 1)) rank_rows(a, reinterpret_cast<int*>(sKV));  // K/V buffers are free here
+    if constexpr (!PIPE) {
+      if (!even) {
+        __syncthreads();  // the ranks are visible
+        run_claims(a, n_items, sKV, sQ, s_ml, s_row, s_mask);
+        return;
+      }
+    }
     const int fixed = LOOKAHEAD * (int)gridDim.x;
     // All items dealt: no workgroup claims, and one looks whether the claims word was zero (read
     // here, looked at after its items, so nothing waits for it).
@@ -1867,7 +1923,6 @@ static hipError_t launch_sub(PrefillArgs a, int64_t n_items, int64_t item_grid, 
   if (a.claims) grid = std::min<int64_t>(n_items, (int64_t)num_cus() * resident_per_cu<BF16, D, HW, NS, SUB>());
   // Queues need claims, owners in equal numbers and LOOKAHEAD items for each.
   if (n_items <= LOOKAHEAD * grid || grid % N_XCD) a.queues = 1;
-  if (a.queues > 1) a.row_order = 0;
   hipLaunchKernelGGL((prefill_kernel<BF16, D, HW, NS, SUB>), dim3(grid), dim3(128 * HW * NS), 0, s, a);
   return hipGetLastError();
 }
@@ -2091,10 +2146,10 @@ static int prefill_impl(const char* fn, int dtype,
   // Queues: one XCD keeps to a few KV heads, whose K/V its L2 can hold (past the L2s the Infinity Cache
   // serves 26-30 B/ns per CU, an L2 117-145).  Items that read a whole KV head's rows one head at a time
   // gain most: 8,192 tokens of 32 heads, blocks of 32, 335 us with one queue, 280 with eight; a window of
-  // 512 175 / 124 us; 32,768 tokens 528 / 449; rows whose lengths differ by a group's budget (2 to 30 %)
-  // 396 / 358.  Four heads to an item read less: dense 8,192 tokens 716 / 604, blocks drawn from 8,192
-  // tokens 319 / 315, and past the L2 nothing: the 32K-token prompt (16 MB per head, groups of different
-  // densities) 335 / 392 us.
+  // 512 175 / 124 us; 32,768 tokens 528 / 449.  Four heads to an item read less: dense 8,192 tokens
+  // 600 / 520, blocks drawn from 8,192 tokens 319 / 315, and past the L2 nothing: the 32K-token prompt (16 MB
+  // per head, groups of different densities) 335 / 392 us.  Rows of different lengths turn them off in the
+  // kernel (rows_even).
   const int64_t heads = (int64_t)B * Hkv, head_bytes = (int64_t)T_k * D * 4;
   constexpr int64_t L2_BYTES = 4 << 20;
   a.queues = 1;

@@ -69,3 +69,11 @@ def _ratio(Hq, rows, B, T, profile, ws_bytes):
 def test_one_queue_four_heads(B, T, profile):
     """Four items per workgroup, the first three dealt by index."""
     assert _ratio(32, 8, B, T, profile, int(_lib.load().sa_prefill_workspace_bytes())) <= SLACK
+
+
+@pytest.mark.parametrize("Hq,rows,B,T", [(32, 8, 1, 8192), (32, 8, 2, 4096), (32, 32, 1, 8192), (32, 32, 4, 4096),
+                                         (16, 8, 2, 8192), (16, 8, 1, 12000)])
+@pytest.mark.parametrize("profile", list(PROFILES))
+def test_queue_workspace(Hq, rows, B, T, profile):
+    """With room for a queue per XCD: four, one and two heads to an item, even and uneven rows."""
+    assert _ratio(Hq, rows, B, T, profile, int(_lib.load().sa_prefill_queue_workspace_bytes())) <= SLACK
