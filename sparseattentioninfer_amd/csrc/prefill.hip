@@ -293,11 +293,12 @@ struct Prefill {
   static constexpr int WAVE_BYTES = QT * D * 2;  // 32 rows of Q or O (one wave's share)
   // Four-head workgroups run the software-pipelined loop with K double- and V triple-
   // buffered and Q staged in LDS.  Other shapes hold one K and one V tile per slice, each refilled
-  // as soon as it has been read (so four two-wave workgroups share a CU); slices merge their
-  // accumulators in fp32 through the same LDS.
+  // as soon as it has been read (so four two-wave workgroups share a CU), or two of each where only
+  // two workgroups share a CU anyway (DB); slices merge their accumulators in fp32 through the same LDS.
   static constexpr bool PIPE = HW == 4;
-  static constexpr int NBK = PIPE ? 2 : 1;
-  static constexpr int NBV = PIPE ? 3 : 1;
+  static constexpr bool DB = HW == 2 && NS == 1;
+  static constexpr int NBK = PIPE || DB ? 2 : 1;
+  static constexpr int NBV = PIPE ? 3 : DB ? 2 : 1;
   static constexpr int LDS_TILES = NS * (NBK + NBV) * TILE_BYTES;
   static constexpr int LDS_MERGE = NS > 1 ? NW * QT * D * 4 : 0;
   static constexpr int LDS_KV = LDS_TILES > LDS_MERGE ? LDS_TILES : LDS_MERGE;
@@ -307,7 +308,7 @@ struct Prefill {
   static constexpr float REFIT_SUM = BF16 ? 65536.f : 32768.f;
   static_assert(NI % TW == 0, "direct loads must split evenly over the waves");
   static_assert(NS == 1 || !PIPE, "four-head workgroups have one slice");
-  static_assert(TW * WAVE_BYTES <= (NBK + NBV) * TILE_BYTES, "the epilogue stages O in the K/V buffers");
+  static_assert(TW * WAVE_BYTES <= (PIPE ? NBK + NBV : 2) * TILE_BYTES, "the epilogue stages O in the K/V buffers");
   static_assert(!KS || PIPE, "key splits are for four-head workgroups");
   static_assert(!TL || PIPE, "the timeline instruments the persistent four-head loop");
 
@@ -1045,8 +1046,11 @@ struct Prefill {
   // the item's usable tiles s, s + NS, ...  A wave whose 32 rows see nothing of a tile (causal limit,
   // sub-block masks) only loads it: with blocks of 16 or 32 the two halves of a query tile keep mostly
   // different blocks.
-  // With one slice four (two) workgroups share a CU and run at different points of their tiles, so a
-  // tile simply waits for its loads.  With slices the CU holds one workgroup (two with NS = 2), and its
+  // With one slice four one-head workgroups share a CU and run at different points of their tiles, so a
+  // tile simply waits for its loads.  Two-head workgroups, two to a CU, load the next tile into the other
+  // buffers under the work on this one, with one barrier per tile: with single buffers a long item alone on
+  // its CU waited for every tile (16 heads, batch 2, one dense KV head of eight: 4,096 tokens 134 us, now
+  // 116, 8,192 tokens 253, now 214; all dense 8,192 tokens 623, now 593).  With slices the CU holds one workgroup (two with NS = 2), and its
   // loads must run under its own work: K is refilled once every wave has read it (under the
   // exponentials and the PV product), V after the PV product (under the next QK product).  That order
   // costs two more barriers per tile and was slower with one slice: 8,192 tokens of 8 heads of 64,
@@ -1064,6 +1068,12 @@ struct Prefill {
     const int w2 = wave % TW;
     char* sK = sKV + slice * 2 * TILE_BYTES;
     char* sV = sK + TILE_BYTES;
+    int buf = 0;  // DB: the pair of buffers that sK and sV are
+    auto flip = [&] {
+      buf ^= 1;
+      sK = sKV + buf * 2 * TILE_BYTES;
+      sV = sK + TILE_BYTES;
+    };
     const Item it = LOOK ? setup_base(a, qt, r, hs, b, lk->e0, lk->n_ent) : setup(a, qt, r, hs, b, s_row, s_mask);
     // Q^T as the B operand of S^T = K Q^T: lane holds row l32, d = 16c + 8g .. +7.
     u32x4 qf[D / 16];
@@ -1191,7 +1201,15 @@ struct Prefill {
       // the row a key and raised only when a lane's probabilities sum past REFIT_SUM or overflow.
       if constexpr (NS == 1) {
         wait_dma();
-        __syncthreads();  // K and V are in LDS
+        __syncthreads();  // K and V are in LDS (and DB: the other buffers have been read)
+        if constexpr (DB) {
+          flip();
+          if (has_n) {
+            load_k(kt_n);
+            load_v(kt_n);
+          }
+          flip();
+        }
         if (active) {
           qk(S);
           if (masked) mask_tile(a, S, row_bits(a, m, it.hf, it.l32), lim0 - kt * KT);
@@ -1208,10 +1226,14 @@ struct Prefill {
             pv(P[j], j);
           }
         }
-        __syncthreads();  // both have been read
-        if (has_n) {
-          load_k(kt_n);
-          load_v(kt_n);
+        if constexpr (DB) {
+          flip();
+        } else {
+          __syncthreads();  // both have been read
+          if (has_n) {
+            load_k(kt_n);
+            load_v(kt_n);
+          }
         }
       } else {
         __builtin_amdgcn_s_waitcnt(0x0F70 | (NIW & 15));  // vmcnt(NIW): K is in LDS, V may be in flight
@@ -1246,9 +1268,10 @@ struct Prefill {
       kt = kt_n;
       m = m_n;
     }
-    // Every wave has passed the last barrier: the K/V buffers are free for the staging.
+    // The K/V buffers are free for the staging: every wave has passed the last barrier, after which DB's
+    // waves read only the pair that is not sK and sV now.
     if constexpr (NS == 1)
-      epilogue(a, it, b, O, l_run, sKV + wave * WAVE_BYTES, lane);
+      epilogue(a, it, b, O, l_run, sKV + buf * 2 * TILE_BYTES + wave * WAVE_BYTES, lane);
     else
       epilogue_slices(a, it, b, O, m_ref, l_run, sKV, s_ml, slice, w2, lane);
   }
@@ -1831,8 +1854,8 @@ struct Prefill {
       if (wave % HW == 0 && (threadIdx.x & 63) == 0) s_tl[wave / HW][TL_NOW] = (unsigned)__builtin_amdgcn_s_memtime();
     }
     // Up to two items per workgroup the second round, which runs in reverse, balances uneven rows as well
-    // as claims do (4,096 tokens of 16 heads, one dense KV head of eight: 118 us dealt, 112 claimed; equal
-    // windows 38 against 44).
+    // as claims do (2 x 4,096 tokens of 16 heads, one dense KV head of eight: 118 us dealt, 112 claimed;
+    // windows of 1 to 12 blocks 41 against 55).
     const bool even = a.queues > 1 || (!PIPE && n_items > 2 * (int)gridDim.x) ? rows_even(a) : true;
     if (threadIdx.x == 0) s_queued = even;
     if (a.row_order && !(even && a.queues > 1)) rank_rows(a, reinterpret_cast<int*>(sKV));  // K/V buffers are free here
