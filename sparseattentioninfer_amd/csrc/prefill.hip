@@ -822,7 +822,8 @@ struct Prefill {
   // it.  Its first LOOKAHEAD items per owner are dealt, the others claimed, so every item is dealt or
   // claimed once: an owner leaves its queue only when the queue has run out.
   enum : int { CL_QUEUE = 0, CL_TAKEN = 1, CL_WORDS = 2 };  // queue claimed from, items taken
-  static __device__ __forceinline__ bool queued(const PrefillArgs& a) { return !KS && a.queues > 1 && s_queued; }
+  static constexpr bool QUEUES = !KS && !TL && NS == 1;  // slices: at most one item per workgroup
+  static __device__ __forceinline__ bool queued(const PrefillArgs& a) { return QUEUES && a.queues > 1 && s_queued; }
   static __device__ __forceinline__ int queue_start(const PrefillArgs& a, int x, int n_items) {
     return queued(a) ? (int)((int64_t)n_items * x / N_XCD) : x * n_items;
   }
@@ -1802,18 +1803,31 @@ struct Prefill {
     }
   }
 
-  // Persistent loop of one- and two-head workgroups over uneven rows: one queue, and every item is
-  // claimed when the one before it has ended.
-  static __device__ __forceinline__ void run_claims(const PrefillArgs& a, int n_items, char* sKV, char* sQ, float* s_ml,
-                                                    int32_t* s_row, int32_t* s_mask) {
-    __shared__ int s_item;
+  // Items one at a time: the workgroup's only one (no workspace), or, for one- and two-head workgroups
+  // over uneven rows, one queue of which every item is claimed when the one before it has ended.
+  static constexpr bool CLAIM_EACH = QUEUES && !PIPE;
+  static __device__ __forceinline__ void run_items(const PrefillArgs& a, int n_items, char* sKV, char* sQ, float* s_ml,
+                                                   int32_t* s_row, int32_t* s_mask) {
     for (int taken = 0;; taken = 1) {
-      if (threadIdx.x == 0) s_item = claimed_item(a.claims, a.status, add_claim(a.claims, taken), taken, 0, n_items);
-      __syncthreads();
-      const int v = s_item;
-      __syncthreads();
-      if (v >= n_items) break;
+      int v;
+      if (!CLAIM_EACH || !a.claims) {
+        // Consecutive workgroups go to the 8 XCDs in turn; chunks of XCD_CHUNK consecutive query tiles
+        // (all rows) are dealt to the XCDs round-robin so every XCD gets an even share of each row's
+        // work, while neighbouring tiles (which share window and global key blocks) stay in one XCD's L2.
+        const int per_tile = a.R * a.B * a.head_splits;
+        const int chunk = XCD_CHUNK * per_tile;
+        const int xcd = blockIdx.x % N_XCD, seq = blockIdx.x / N_XCD;
+        v = ((seq / chunk) * N_XCD + xcd) * chunk + seq % chunk;
+      } else {
+        __shared__ int s_item;
+        if (threadIdx.x == 0) s_item = claimed_item(a.claims, a.status, add_claim(a.claims, taken), taken, 0, n_items);
+        __syncthreads();
+        v = s_item;
+        __syncthreads();
+      }
+      if (v >= n_items) break;  // none left, or a padding workgroup of the last round
       process(a, v, sKV, sQ, s_ml, s_row, s_mask);
+      if (!CLAIM_EACH || !a.claims) break;
     }
   }
 
@@ -1826,21 +1840,6 @@ struct Prefill {
     __shared__ int32_t s_mask[SUB ? 2 * RC : 1];  // sub-block masks of the cached rows
     const int n_items = a.ntq * a.R * a.B * a.head_splits * (KS ? a.splits : 1);
 
-    if (!a.claims) {
-      // One workgroup per item.  Consecutive workgroups go to the 8 XCDs in turn; chunks of
-      // XCD_CHUNK consecutive query tiles (all rows) are dealt to the XCDs round-robin so every
-      // XCD gets an even share of each row's work, while neighbouring tiles (which share
-      // window and global key blocks) stay in one XCD's L2.
-      const int per_tile = a.R * a.B * a.head_splits;
-      const int chunk = XCD_CHUNK * per_tile;
-      const int xcd = blockIdx.x % N_XCD, seq = blockIdx.x / N_XCD;
-      const int v = ((seq / chunk) * N_XCD + xcd) * chunk + seq % chunk;
-      if (v >= n_items) return;  // padding workgroup of the last round
-      process(a, v, sKV, sQ, s_ml, s_row, s_mask);
-      return;
-    }
-
-    // Persistent: the dealt items, then claims until one fails.
     unsigned long long* rec = nullptr;  // TL: this workgroup's record
     if constexpr (TL) {
       rec = a.timeline + (int64_t)blockIdx.x * TL_WORDS;
@@ -1853,19 +1852,26 @@ struct Prefill {
       const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
       if (wave % HW == 0 && (threadIdx.x & 63) == 0) s_tl[wave / HW][TL_NOW] = (unsigned)__builtin_amdgcn_s_memtime();
     }
-    // Up to two items per workgroup the second round, which runs in reverse, balances uneven rows as well
-    // as claims do (2 x 4,096 tokens of 16 heads, one dense KV head of eight: 118 us dealt, 112 claimed;
-    // windows of 1 to 12 blocks 41 against 55).
-    const bool even = a.queues > 1 || (!PIPE && n_items > 2 * (int)gridDim.x) ? rows_even(a) : true;
-    if (threadIdx.x == 0) s_queued = even;
-    if (a.row_order && !(even && a.queues > 1)) rank_rows(a, reinterpret_cast<int*>(sKV));  // K/V buffers are free here
-    if constexpr (!PIPE) {
-      if (!even) {
+    bool dealt = a.claims;
+    if (dealt) {
+      // Up to two items per workgroup the second round, which runs in reverse, balances uneven rows as well
+      // as claims do (2 x 4,096 tokens of 16 heads, one dense KV head of eight: 118 us dealt, 112 claimed;
+      // windows of 1 to 12 blocks 41 against 55).
+      const bool queues = QUEUES && a.queues > 1;
+      const bool even = queues || (CLAIM_EACH && n_items > 2 * (int)gridDim.x) ? rows_even(a) : true;
+      if (queues && threadIdx.x == 0) s_queued = even;
+      if (a.row_order && !(queues && even)) rank_rows(a, reinterpret_cast<int*>(sKV));  // K/V buffers are free here
+      if (CLAIM_EACH && !even) {
         __syncthreads();  // the ranks are visible
-        run_claims(a, n_items, sKV, sQ, s_ml, s_row, s_mask);
-        return;
+        dealt = false;
       }
     }
+    if (!dealt) {
+      run_items(a, n_items, sKV, sQ, s_ml, s_row, s_mask);
+      return;
+    }
+
+    // Persistent: the dealt items, then claims until one fails.
     const int fixed = LOOKAHEAD * (int)gridDim.x;
     // All items dealt: no workgroup claims, and one looks whether the claims word was zero (read
     // here, looked at after its items, so nothing waits for it).
@@ -2177,7 +2183,7 @@ static int prefill_impl(const char* fn, int dtype,
   constexpr int64_t L2_BYTES = 4 << 20;
   a.queues = 1;
   if (workspace && workspace_bytes >= WS_QUEUE_BYTES && (reinterpret_cast<uintptr_t>(workspace) & 7) == 0 && !timeline &&
-      a.splits == 1 && heads % N_XCD == 0 && (hw < 4 || head_bytes <= L2_BYTES))
+      a.splits == 1 && ns == 1 && heads % N_XCD == 0 && (hw < 4 || head_bytes <= L2_BYTES))
     a.queues = N_XCD;
   a.unit_heads = 1;  // the largest divisor of a queue's heads that fits
   for (int64_t g = 2; g <= heads / N_XCD && g * head_bytes <= L2_BYTES; ++g)
