@@ -2011,7 +2011,9 @@ static int64_t timeline_grid(bool bf16) {
 //   (512 waves); 2,048 queries 178.7 / 126.8 / 138.3 (1,024 waves), 4,096 queries 265.7 / 263.5 / 427.7;
 //   four heads, 512 queries on 4,512 keys (512 waves): 97.9 pipelined, 62.7 with (1, 4); 1,000 queries
 //   114.7 / 127.7; BigBird of 8 tiles, 512 tokens (512 waves) 17.5 / 13.4, 1,000 tokens 18.8 / 23.9.
-// Four-head launches with at most 15 key tiles stay pipelined: there is little to divide.
+// Four-head launches with at most 15 key tiles stay pipelined, and smaller ones with at most two unsliced:
+// there is little to divide.  40 tokens of 16 heads of 128 7.9 us with (2, 1), 10.2 with (1, 4), 128 tokens
+// 9.7 / 10.8; of 8 heads of 64 7.0 / 8.1 with (1, 1) / (1, 4), 128 tokens 7.9 / 8.2.
 struct Shape {
   int hw, ns;
 };
@@ -2023,8 +2025,9 @@ static Shape choose_shape(int T_q, int T_k, int rows, int B, int heads_per_row) 
     if (waves <= 2 * cus && T_k > 15 * KT) return {1, 4};
     return {4, 1};
   }
-  if (waves <= 2 * cus) return {1, 4};
   const int hw = heads_per_row % 2 == 0 ? 2 : 1;
+  if (T_k <= 2 * KT) return {hw, 1};
+  if (waves <= 2 * cus) return {1, 4};
   return {hw, waves <= 4 * cus ? 2 : 1};
 }
 

@@ -10,6 +10,7 @@ import torch
 from oracle import attention as oa
 from sparseattentioninfer_amd import ops
 from sparseattentioninfer_amd.patterns import bernoulli_block_mask, block_mask_to_csr
+from tests.helpers import assert_close_bf16, seeded
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -44,3 +45,19 @@ def test_shapes_match_the_oracle(per_cu, heads, kv, rows, D, bs, T_q, T_k, dtype
     bound = u * v.float().abs().amax() + 2 * u * want.to(out.device).abs() + 2e-3
     assert (err <= bound).all(), f"max-abs {err.max():.3e}, {(err / bound).max():.2f} of the bound"
     assert err.mean() <= 2e-3
+
+
+@pytest.mark.parametrize("heads,kv,rows", [(4, 2, 2), (4, 4, 4), (4, 1, 1)])
+@pytest.mark.parametrize("D,bs,T_q,T_k", [(128, 64, 40, 40), (64, 16, 2, 33), (128, 64, 300, 300), (64, 64, 70, 2118),
+                                          (128, 128, 200, 200)])
+def test_lists_of_one_tile_match_the_oracle(heads, kv, rows, D, bs, T_q, T_k):
+    """Few items, diagonal blocks only (one tile per item, or two with blocks of 128)."""
+    print(f"[prefill shapes] one tile: heads={heads}/{kv} rows={rows} D={D} bs={bs} T={T_q}/{T_k}", flush=True)
+    sys.stdout.flush()
+    nqb, nkb = -(-T_q // bs), -(-T_k // bs)
+    bm = (torch.arange(nkb)[None] == torch.arange(nqb)[:, None] + (T_k - T_q) // bs).expand(rows, -1, -1)
+    pairs, offsets = block_mask_to_csr(bm)
+    q = seeded((2, heads, T_q, D), 1, torch.bfloat16)
+    k, v = (seeded((2, kv, T_k, D), s, torch.bfloat16) for s in (2, 3))
+    out = ops.universal_sparse_attn(q.to(DEV), k.to(DEV), v.to(DEV), pairs.to(DEV), offsets.to(DEV), bs)
+    assert_close_bf16(out, oa.block_sparse_attention(q, k, v, pairs, offsets, bs), "one tile")
