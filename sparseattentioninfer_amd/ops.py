@@ -418,7 +418,8 @@ def paged_sparse_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.T
     [B, R, 2]`` int32 retained logical blocks per (sequence, row), R = Hq or
     Hkv.  ``num_splits > 1`` splits each row over workgroups and needs a
     byte workspace of :func:`decode_workspace_bytes` (allocated if omitted);
-    ``num_splits=0`` picks the count from the shapes.
+    ``num_splits=0`` picks the count from the shapes: :func:`decode_splits`, or, with a workspace
+    too small for that, :func:`auto_decode_splits`.
     """
     name = "paged_sparse_decode"
     q3 = q.reshape(q.shape[0], q.shape[1], q.shape[-1]) if q.dim() == 4 else q
@@ -457,6 +458,9 @@ def paged_sparse_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.T
     Hkv, page = k_pages.size(1), k_pages.size(2)
     if num_splits == 0:
         num_splits = decode_splits(B, Hq, R, sel.shape[2])
+        if workspace is not None and \
+                workspace.numel() * workspace.element_size() < decode_workspace_bytes(B, Hq, D, num_splits):
+            num_splits = auto_decode_splits(B, R, sel.shape[2])     # a workspace sized with its count serves
     if out is None:
         out = torch.empty(B, Hq, D, dtype=q3.dtype, device=q3.device)
     lib = _lib.load()

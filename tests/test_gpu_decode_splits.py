@@ -42,3 +42,24 @@ def test_split_decode_matches_the_oracle(B, Hq, Hkv, rows, D, bs, T, dtype):
                                   pairs.to(DEV)[None].expand(B, -1, -1), offsets.to(DEV)[None].expand(B, -1, -1),
                                   num_splits=0)
     assert_close_bf16(got, want, "paged")
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,n", [(1, 32, 8, 100), (1, 8, 2, 64), (8, 32, 8, 27)])
+def test_chosen_split_count_fits_a_workspace_of_either_rule(B, Hq, Hkv, n):
+    """``num_splits=0`` with a caller's workspace, sized by either public count."""
+    D, page = 128, 16
+    print(f"[decode splits] workspace: B={B} heads={Hq}/{Hkv} {n} blocks", flush=True)
+    sys.stdout.flush()
+    q = seeded((B, Hq, D), 1, torch.bfloat16).to(DEV)
+    kp, vp = (seeded((B * n, Hkv, page, D), s, torch.bfloat16).to(DEV) for s in (2, 3))
+    table = torch.arange(B * n, dtype=torch.int32, device=DEV).reshape(B, n)
+    lens = torch.full((B,), n * page, dtype=torch.int32, device=DEV)
+    sel = torch.arange(n, dtype=torch.int32, device=DEV).expand(B, Hkv, n).contiguous()
+    off = torch.tensor([0, n], dtype=torch.int32, device=DEV).expand(B, Hkv, 2).contiguous()
+    args = (q, kp, vp, table, lens, sel, off)
+    for splits in (ops.auto_decode_splits(B, Hkv, n), ops.decode_splits(B, Hq, Hkv, n)):
+        ws = torch.empty(ops.decode_workspace_bytes(B, Hq, D, splits), dtype=torch.uint8, device=DEV)
+        got = ops.paged_sparse_decode(*args, num_splits=0, workspace=ws)
+        assert_close_bf16(got, ops.paged_sparse_decode(*args), "workspace")
+    with pytest.raises(AssertionError, match="workspace too small"):
+        ops.paged_sparse_decode(*args, num_splits=0, workspace=ws[:1024])
