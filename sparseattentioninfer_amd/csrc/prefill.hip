@@ -862,6 +862,18 @@ struct Prefill {
     return n < (unsigned)(queue_start(a, x + 1, n_items) - s) ? s + (int)n : n_items;
   }
 
+  // Adds one and `taken` to a finish word; the last of `count` zeroes it, gets the sum of the taken and
+  // returns true.  A word that has counted more than `count` was not zero at launch: no one is the last.
+  static __device__ __forceinline__ bool last_of(const PrefillArgs& a, unsigned long long* word, unsigned count,
+                                                 unsigned long long& taken) {
+    const unsigned long long old = atomicAdd(word, 1ull | (taken << 32));
+    if ((unsigned)old >= count) atomicOr(a.status, WS_SKIPPED);
+    if ((unsigned)old != count - 1) return false;
+    atomicExch(word, 0ull);
+    taken += old >> 32;
+    return true;
+  }
+
   // Thread 0: the item of the claim that read n from the current queue, or n_items (see WS_CLAIMS).
   // Once a queue has run out, each of its owners looks at one of the other seven, by its index (all of
   // them looking at all seven counters costs more than it balances, 1,024 workgroups on 8 lines: 8,192
@@ -883,14 +895,8 @@ struct Prefill {
       return v;
     }
     unsigned long long taken = (unsigned)cl[CL_TAKEN];
-    unsigned long long old = atomicAdd(&a.claims[own * WS_QUEUE + WS_FINISH], 1ull | (taken << 32));
-    if ((unsigned)old != (unsigned)owners(a) - 1) return n_items;
-    atomicExch(&a.claims[own * WS_QUEUE + WS_FINISH], 0ull);
-    taken += old >> 32;
-    old = atomicAdd(&a.claims[WS_ALL], 1ull | (taken << 32));
-    if ((unsigned)old != N_XCD - 1) return n_items;
-    atomicExch(&a.claims[WS_ALL], 0ull);
-    taken += old >> 32;
+    if (!last_of(a, &a.claims[own * WS_QUEUE + WS_FINISH], (unsigned)owners(a), taken)) return n_items;
+    if (!last_of(a, &a.claims[WS_ALL], N_XCD, taken)) return n_items;
     bool ok = taken == (unsigned long long)n_items;
     for (int y = 0; y < N_XCD; ++y) ok = (atomicExch(&a.claims[y * WS_QUEUE + WS_CLAIMS], 0ull) >> 32) == 0 && ok;
     if (!ok) atomicOr(a.status, WS_SKIPPED);

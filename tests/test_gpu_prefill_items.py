@@ -8,7 +8,7 @@ import sys
 import pytest
 import torch
 
-from sparseattentioninfer_amd import _lib
+from sparseattentioninfer_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -28,16 +28,28 @@ def _case(n, rows):
     return q, k, v, flat.expand(R, -1).contiguous().to(DEV), offsets.expand(R, -1).contiguous().to(DEV), R, 64
 
 
-def _launch(q, k, v, pairs, offsets, R, bs, ws):
+def _windows(B, Hq, Hkv, T, D, windows):
+    """Row r keeps the last ``windows[r]`` blocks of 64 keys."""
+    n = -(-T // 64)
+    g = torch.Generator(device=DEV).manual_seed(n)
+    q = torch.randn(B, Hq, T, D, generator=g, device=DEV).bfloat16()
+    k, v = (torch.randn(B, Hkv, T, D, generator=g, device=DEV).bfloat16() for _ in range(2))
+    qb, kb = torch.arange(n, device=DEV)[:, None], torch.arange(n, device=DEV)[None]
+    pairs, offsets = ops.block_mask_to_csr_gpu(torch.stack([(kb <= qb) & (kb > qb - w) for w in windows]))
+    return q, k, v, pairs, offsets
+
+
+def _launch(q, k, v, pairs, offsets, R, bs, ws, split=False):
+    """``sa_prefill``, or with ``split`` ``sa_prefill_split`` (queues, in a workspace with room for them)."""
     lib = _lib.load()
     o = torch.full_like(q, float("nan"))
     B, Hq, T, D = q.shape
-    st = lib.sa_prefill(0, q.data_ptr(), *q.stride()[:3], k.data_ptr(), *k.stride()[:3], v.data_ptr(), *v.stride()[:3],
-                        o.data_ptr(), *o.stride()[:3], pairs.data_ptr(), pairs.stride(0), offsets.data_ptr(),
-                        offsets.stride(0), None, 0, R, offsets.size(1) - 1, B, Hq, k.shape[1], T, T, D, bs, 0,
-                        1.0 / math.sqrt(D), ws.data_ptr() if ws is not None else None,
-                        4 * ws.numel() if ws is not None else 0,
-                        torch.cuda.current_stream().cuda_stream)
+    fn, partials = (lib.sa_prefill_split, (None, 0)) if split else (lib.sa_prefill, ())
+    st = fn(0, q.data_ptr(), *q.stride()[:3], k.data_ptr(), *k.stride()[:3], v.data_ptr(), *v.stride()[:3],
+            o.data_ptr(), *o.stride()[:3], pairs.data_ptr(), pairs.stride(0), offsets.data_ptr(),
+            offsets.stride(0), None, 0, R, offsets.size(1) - 1, B, Hq, k.shape[1], T, T, D, bs, 0,
+            1.0 / math.sqrt(D), ws.data_ptr() if ws is not None else None,
+            4 * ws.numel() if ws is not None else 0, *partials, torch.cuda.current_stream().cuda_stream)
     assert st == 0, lib.sa_last_error()
     return o
 
@@ -93,40 +105,64 @@ def test_workspace_aligned_to_four_bytes_only():
         assert torch.equal(got, want)
 
 
-@pytest.mark.parametrize("Hq,Hkv,rows,B", [(16, 8, 16, 1), (8, 8, 8, 2), (32, 8, 8, 1), (12, 4, 12, 2), (6, 6, 6, 4), (24, 8, 24, 3)])
-@pytest.mark.parametrize("skew", [False, True])
-def test_queues_per_xcd_process_every_item_once(Hq, Hkv, rows, B, skew):
-    """Launches with claims and a KV-head count that the XCDs divide evenly (or not: one queue then), even
-    and skewed row lengths (queues that run out early claim from the others): the bits of the launch
-    without a workspace, and a workspace that is zero afterwards."""
+FINISH, ALL, QUEUE = 2, 4, 16      # 64-bit words of a queue workspace: a queue's finish word, the queues', per queue
+
+
+@pytest.mark.parametrize("Hq,Hkv,rows,B,D,T", [
+    (16, 8, 16, 1, 64, 32759), (8, 8, 8, 2, 64, 32759), (24, 8, 24, 3, 64, 7295),       # one head to an item
+    (16, 8, 8, 8, 64, 4091), (16, 8, 8, 6, 128, 4091),                                  # two, units of four and two heads
+    (32, 8, 8, 4, 64, 4091), (32, 8, 8, 4, 128, 4091), (64, 8, 8, 2, 128, 4091),        # four; two items per head
+    (32, 8, 8, 1, 128, 16379), (20, 5, 5, 4, 128, 4091), (5, 5, 5, 20, 64, 4091),       # one queue: K/V past the L2; 20 heads
+    (12, 4, 12, 2, 64, 21832), (6, 6, 6, 4, 64, 21832)])
+@pytest.mark.parametrize("windows", ["even", "nearly", "uneven"])
+def test_queues_per_xcd_process_every_item_once(Hq, Hkv, rows, B, D, T, windows):
+    """Launches with claims, with and without a queue per XCD, rows of one length, of nearly one (queues that
+    run out early claim from others) and of very different ones: the bits of the launch without a
+    workspace, and a workspace that is zero afterwards.  Whether a launch used queues shows in a finish
+    word that was not zero, which only they look at."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    per_item = 4 if Hq // rows == 4 else 1
-    n = -(-(8 if per_item == 1 else 4) * 4 * cus * per_item // (Hq * B))     # query tiles: several items per workgroup
-    D, bs, T = 64, 64, 64 * n - 9
-    print(f"[prefill items] queues: heads {Hq}/{Hkv} rows {rows} B={B} T={T} skew={skew}", flush=True)
+    per_row = Hq // rows
+    heads = 4 if per_row % 4 == 0 else 2 if per_row % 2 == 0 else 1
+    items = -(-T // 64) * rows * B * per_row // heads
+    assert items > 3 * cus * {1: 6, 2: 3, 4: 1}[heads]         # more than the dealt ones at any occupancy
+    queues = B * Hkv % 8 == 0 and (heads < 4 or T * D * 4 <= 4 << 20) and windows != "uneven"
+    print(f"[prefill items] queues: heads {Hq}/{Hkv} rows {rows} B={B} D={D} T={T} {windows}: {queues}", flush=True)
     sys.stdout.flush()
-    g = torch.Generator(device=DEV).manual_seed(n)
-    q = torch.randn(B, Hq, T, D, generator=g, device=DEV).bfloat16()
-    k, v = (torch.randn(B, Hkv, T, D, generator=g, device=DEV).bfloat16() for _ in range(2))
-    qb = torch.arange(n)
-    lists = []
-    for r in range(rows):
-        w = (1 + 12 * r // rows) if skew else 2                               # blocks of the window
-        lists.append([list(range(max(0, int(i) - w + 1), int(i) + 1)) for i in qb])
-    width = max(sum(map(len, row)) for row in lists)
-    pairs = torch.zeros(rows, width, dtype=torch.int32)
-    offsets = torch.zeros(rows, n + 1, dtype=torch.int32)
-    for r, row in enumerate(lists):
-        flat = [x for e in row for x in e]
-        pairs[r, :len(flat)] = torch.tensor(flat, dtype=torch.int32)
-        offsets[r, 1:] = torch.tensor([len(e) for e in row]).cumsum(0)
-    case = (q, k, v, pairs.to(DEV), offsets.to(DEV), rows, bs)
-    nbytes = int(_lib.load().sa_prefill_queue_workspace_bytes())
-    ws = torch.zeros(nbytes // 4, dtype=torch.int32, device=DEV)
+    w = {"even": [2] * rows, "nearly": [21 if r == rows // 2 else 20 for r in range(rows)],
+         "uneven": [1 + 12 * r // rows for r in range(rows)]}[windows]
+    case = (*_windows(B, Hq, Hkv, T, D, w), rows, 64)
+    ws = torch.zeros(int(_lib.load().sa_prefill_queue_workspace_bytes()) // 4, dtype=torch.int32, device=DEV)
     want = _launch(*case, None)
     for _ in range(3):
-        got = _launch(*case, ws)
+        got = _launch(*case, ws, split=True)
         torch.cuda.synchronize()
         assert not ws.any()
         assert torch.equal(got, want)
     assert torch.isfinite(want.float()).all()
+    ws.view(torch.int64)[5 * QUEUE + FINISH] = 1 << 20
+    got = _launch(*case, ws, split=True)
+    torch.cuda.synchronize()
+    assert int(ws[3]) == int(queues)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("word,value", [(5 * QUEUE, 2), (0, 1 << 20), (3 * QUEUE, 1 << 33), (FINISH, 1 << 20),
+                                        (7 * QUEUE + FINISH, 3), (2 * QUEUE + FINISH, 1 << 33), (ALL, 8), (ALL, 3),
+                                        (ALL, 1 << 33)])
+def test_queue_words_that_were_not_zero_are_reported(word, value):
+    """A claims or finish word of a queue, or the queues' finish word: the status bit is set, and a
+    workspace zeroed afterwards serves the next launch."""
+    print(f"[prefill items] queue word {word} = {value}", flush=True)
+    sys.stdout.flush()
+    case = (*_windows(4, 32, 8, 4091, 64, [3] * 8), 8, 64)
+    ws = torch.zeros(int(_lib.load().sa_prefill_queue_workspace_bytes()) // 4, dtype=torch.int32, device=DEV)
+    want = _launch(*case, None)
+    ws.view(torch.int64)[word] = value
+    _launch(*case, ws, split=True)
+    torch.cuda.synchronize()
+    assert int(ws[3]) == 1
+    ws.zero_()
+    got = _launch(*case, ws, split=True)
+    torch.cuda.synchronize()
+    assert not ws.any()
+    assert torch.equal(got, want)
