@@ -79,18 +79,18 @@ const char* sa_last_error(void);
  * head_dim D: 64 or 128.  nqb = number of CSR query blocks (offsets has
  * nqb + 1 entries per row), nqb == ceil(T_q / max(block_size, 64)).
  *
- * workspace (optional, sa_prefill_workspace_bytes() bytes, 4-byte aligned):
- * with it the kernel runs one persistent workgroup per resident slot that
- * takes its first work items by index and claims the others from counters in
- * the workspace.  It must be zeroed before
+ * workspace (optional, sa_prefill_workspace_bytes() bytes, 4-byte aligned;
+ * bytes past those are not touched): with it the kernel runs one persistent
+ * workgroup per resident slot that takes its first work items by index and
+ * claims the others from counters in the workspace.  It must be zeroed before
  * its first use; every completed launch leaves its counters zeroed again.
  * Launches that may run concurrently (other streams, graph replays on other
  * streams) must not share one workspace: keep one per stream.  Word 3 of the
  * workspace is a status word that launches only set and the caller clears:
  * bit 0 means a launch's counters were not zero at launch or an overlapping
  * launch shared them: it may have processed fewer work items than it has and
- * left the skipped items' outputs unwritten; zero the whole workspace then.  NULL launches one workgroup per work
- * item instead.
+ * left the skipped items' outputs unwritten; zero the whole workspace then.
+ * NULL launches one workgroup per work item instead.
  */
 int sa_prefill(int dtype,
                const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st,
@@ -112,8 +112,11 @@ int sa_prefill(int dtype,
  * workspace), launches whose query tiles are few and whose block lists are
  * long divide each query tile's keys over several workgroups and merge their
  * fp32 partials with a second kernel.  Without it, or where that function
- * returns 0, it is sa_prefill.  Calls that may run concurrently need a buffer
- * each.
+ * returns 0, the launch is sa_prefill's.  Calls that may run concurrently need
+ * a buffer each.  A workspace of sa_prefill_queue_workspace_bytes() bytes or
+ * more that is 8-byte aligned also holds a work queue per XCD, with which
+ * launches may keep the work of a KV head on one XCD: all of those bytes must
+ * be zeroed before the first use then, and are zero again after each launch.
  */
 int sa_prefill_split(int dtype,
                      const void* q, int64_t q_sb, int64_t q_sh, int64_t q_st,
@@ -138,9 +141,7 @@ int64_t sa_prefill_partial_bytes(int csr_rows, int B, int Hq, int T_q, int T_k, 
 /* Bytes of the optional sa_prefill workspace (counters and the status word). */
 int64_t sa_prefill_workspace_bytes(void);
 
-/* Bytes of a sa_prefill workspace that also holds one work queue per XCD: with
- * these (8-byte aligned), launches may keep the work of a KV head on one XCD.
- * Otherwise it is used as a workspace of sa_prefill_workspace_bytes(). */
+/* Bytes of a sa_prefill_split workspace that also holds one work queue per XCD. */
 int64_t sa_prefill_queue_workspace_bytes(void);
 
 /*

@@ -2254,7 +2254,8 @@ extern "C" int sa_prefill(int dtype,
   return sa::prefill_impl("sa_prefill", dtype, q, q_sb, q_sh, q_st, k, k_sb, k_sh, k_st, v, v_sb, v_sh, v_st,
                           o, o_sb, o_sh, o_st, pairs, pairs_stride, offsets, offsets_stride, tile_masks,
                           tile_masks_stride, csr_rows, nqb, B, Hq, Hkv, T_q, T_k, D, block_size, q_offset,
-                          sm_scale, workspace, workspace_bytes, nullptr, 0, stream, nullptr, 0);
+                          sm_scale, workspace, std::min(workspace_bytes, sa_prefill_workspace_bytes()), nullptr, 0,
+                          stream, nullptr, 0);
 }
 
 extern "C" int sa_prefill_split(int dtype,

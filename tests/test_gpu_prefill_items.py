@@ -94,6 +94,21 @@ def test_claims_word_that_was_not_zero_is_reported(rows, rounds, word, value):
     assert torch.equal(got, want)
 
 
+def test_only_the_workspace_bytes_of_a_larger_buffer_are_used():
+    """``sa_prefill`` asks for its 32 bytes to be zero, whatever the size of the buffer they are in."""
+    T, Hkv, B = 4091, 8, 12
+    print("[prefill items] larger buffer", flush=True)
+    q, k, v, pairs, offsets = _windows(B, 8, Hkv, T, 64, [2] * 8)
+    buf = torch.full((1024,), 0x5a5a5a5a, dtype=torch.int32, device=DEV)
+    buf[:8] = 0
+    want = _launch(q, k, v, pairs, offsets, Hkv, 64, None)
+    for _ in range(2):
+        got = _launch(q, k, v, pairs, offsets, Hkv, 64, buf)
+        torch.cuda.synchronize()
+        assert not buf[:8].any() and (buf[8:] == 0x5a5a5a5a).all()
+        assert torch.equal(got, want)
+
+
 def test_workspace_aligned_to_four_bytes_only():
     case = _case(5 * torch.cuda.get_device_properties(0).multi_processor_count + 3, "group")
     buf = torch.zeros(16, dtype=torch.int32, device=DEV)
