@@ -2106,6 +2106,7 @@ static int prefill_impl(const char* fn, int dtype,
     if (s % 8) return set_error(SA_E_ALIGN, "%s: stride %lld is not a multiple of 8 elements", fn, (long long)s);
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o))
     return set_error(SA_E_ALIGN, "%s: tensor base pointers must be 16-byte aligned", fn);
+  if (!aligned16(partials)) return set_error(SA_E_ALIGN, "%s: partials must be 16-byte aligned", fn);
   if (k_st < 0 || v_st < 0 || k_st > MAX_KV_STRIDE || v_st > MAX_KV_STRIDE)
     return set_error(SA_E_SHAPE, "%s: K/V token strides %lld, %lld outside [0, %lld]", fn, (long long)k_st,
                      (long long)v_st, (long long)MAX_KV_STRIDE);

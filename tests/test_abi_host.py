@@ -78,6 +78,10 @@ def test_argument_errors_are_reported_without_a_gpu(lib):
     assert lib.sa_decode_workspace_bytes(2, 4, 128, 3) == 3 * 2 * 4 * 130 * 4
     assert lib.sa_decode_workspace_bytes(2, 4, 128, 1) == 0
     assert lib.sa_prefill_workspace_bytes() == 32            # counters and the status word (word 3)
+    # the partial results of a divided prefill are accessed 16 bytes at a time
+    st = lib.sa_prefill_split(0, fake, 8, 8, 8, fake, 8, 8, 8, fake, 8, 8, 8, fake, 8, 8, 8, fake, 8, fake, 8, None, 0,
+                              2, 2, 1, 8, 2, 100, 100, 128, 64, 0, 0.1, fake, 32, fake + 4, 1 << 20, None)
+    assert st == -8 and b"partials must be 16-byte aligned" in lib.sa_last_error()
     # the no-allocation decode refuses sizes past its scratch array before anything else (NULL tensors:
     # a call let through would stop at sa_decode's own NULL check, a different status)
     cap = int(lib.sa_decode_noalloc_scratch_bytes())
