@@ -383,7 +383,8 @@ def decode_workspace_bytes(B: int, Hq: int, D: int, num_splits: int) -> int:
 
 def auto_decode_splits(B: int, rows: int, max_sel: int, target_workgroups: int = 512) -> int:
     """Splits of each (sequence, row) block list so that a decode launch has about
-    ``target_workgroups`` workgroups (two per CU), keeping at least two blocks per split."""
+    ``target_workgroups`` workgroups (two per CU), keeping at least two blocks per split.  It knows
+    nothing of the heads; :func:`decode_splits` does, and is what ``num_splits=0`` and the graph decoder use."""
     base = max(1, B * rows)
     want = -(-target_workgroups // base)
     return max(1, min(want, max_sel // 2, 16))
@@ -399,10 +400,29 @@ def decode_splits(B: int, Hq: int, rows: int, max_sel: int) -> int:
     workgroups unsplit, 134 MB) 41.7 / 27.1 / 28.5 / 34.2 with 4 / 8 / 16 / 32 splits; one of 32,000 (8)
     72.9 / 42.0 / 28.8 / 31.9 with 8 / 16 / 32 / 64; 14 blocks of 64 kept by 64 workgroups 19.5 / 15.3 /
     13.3 / 13.2 with 1 / 2 / 4 / 8, by 128 20.1 / 17.6 / 19.0 with 1 / 2 / 4, by 192 22.0 / 25.2 with 1 / 2.
+
+    Workgroups of fewer than four heads that read the same list (groups of 3, 6 or 7 heads) each draw its
+    keys, from their XCD's L2 if their splits, which are numbered first, are a multiple of its eight.  Long
+    lists then take 8 or 16 splits (blocks of 64; 1 to 2 splits, 8, 16): 96 workgroups of one head on 64
+    blocks 28.2 / 27.4 / 25.1, 192 on 40 blocks 30.9 / 27.2, 288 on 64 blocks 80.5 / 62.5 (6 splits 67.3),
+    192 of two heads on 128 blocks 106.5 / 83.3.  Up to 128 workgroups of one head with lists of their own
+    two to a CU are as good or better (96 on 27 blocks 20.2 / 18.8 with 2 / 5, on 8 blocks 11.2 / 9.4).
     """
     per_row = Hq // rows
-    units = B * rows * (per_row // 4 if per_row % 4 == 0 else per_row // 2 if per_row % 2 == 0 else per_row)
-    return max(1, min(256 // max(1, units), max_sel // 2, 32))
+    heads = 4 if per_row % 4 == 0 else 2 if per_row % 2 == 0 else 1       # of one workgroup
+    units = B * rows * (per_row // heads)                                 # workgroups unsplit
+    splits = 256 // max(1, units)
+    if heads < 4 and splits <= 2:
+        if per_row > heads:
+            if units > 128:
+                splits = 8 if max_sel >= (24 if heads == 1 else 32) else splits
+            elif max_sel >= 64:
+                splits = 16
+            elif max_sel >= 32 and heads == 1:
+                splits = 8
+        elif heads == 1 and units <= 128:
+            splits = 512 // units
+    return max(1, min(splits, max_sel // 2, 32))
 
 
 def paged_sparse_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
