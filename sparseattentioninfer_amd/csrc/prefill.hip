@@ -35,7 +35,9 @@
 //    workgroups, whose fp32 partials a second kernel merges;
 //  * with a workspace, one persistent workgroup per CU slot takes its first work items by its
 //    own index and claims further ones from an atomic counter, heaviest query tiles first --
-//    or, where a KV head's K/V fit an L2, from the counter of its XCD's queue of KV heads.
+//    or, where a KV head's K/V fit an L2 and the CSR rows are of about one length, from the counter
+//    of its XCD's queue of KV heads.  One- and two-head workgroups over rows of different lengths
+//    claim every item.
 //
 // MFMA 32x32x16 lane layouts used (l = lane, g = l / 32):
 //   A (32 x 16): lane l holds row l % 32, k = 8g .. 8g+7
@@ -59,7 +61,7 @@ constexpr int XCD_CHUNK = 4;     // query tiles per chunk dealt to one XCD
 // Largest token stride (elements) of K and V: per-lane offsets within a tile are 32-bit.
 constexpr int64_t MAX_KV_STRIDE = (int64_t)1 << 24;
 
-constexpr int LOOKAHEAD = 3;     // items a four-head workgroup holds before it claims from the counter
+constexpr int LOOKAHEAD = 3;     // items dealt to a persistent workgroup by its index, before it claims
 
 struct PrefillArgs {
   const elem_t* q;
@@ -135,9 +137,9 @@ struct PrefillArgs {
 //    fails tries one other queue, and has finished when that gives nothing either.  A finish word
 //    counts its queue's owners that have finished (low half) and the items they have taken (high half);
 //    the last owner passes the sum on, and the last queue's zeroes every word; the items must be all.
-// The items are not all when a word was not zero at launch or launches that overlapped in time shared
-// the words: WS_SKIPPED is set, items may have been skipped and their outputs not written, so the
-// caller must not use the output and zeroes the workspace.
+// The items are not all, or a word counts past its last, when a word was not zero at launch or launches
+// that overlapped in time shared the words: WS_SKIPPED is set, items may have been skipped and their
+// outputs not written, so the caller must not use the output and zeroes the workspace.
 // A workgroup's last claim comes while it still has items to run, so nothing of this is at the end of
 // a launch.  (Two returning atomics on one line and two device-wide fences at the end of every
 // workgroup: 1,024 one-head items of 9 tiles ran 69 us, now 36 us.)
@@ -1057,15 +1059,15 @@ struct Prefill {
   // tile simply waits for its loads.  Two-head workgroups, two to a CU, load the next tile into the other
   // buffers under the work on this one, with one barrier per tile: with single buffers a long item alone on
   // its CU waited for every tile (16 heads, batch 2, one dense KV head of eight: 4,096 tokens 134 us, now
-  // 116, 8,192 tokens 253, now 214; all dense 8,192 tokens 623, now 593).  With slices the CU holds one workgroup (two with NS = 2), and its
-  // loads must run under its own work: K is refilled once every wave has read it (under the
-  // exponentials and the PV product), V after the PV product (under the next QK product).  That order
-  // costs two more barriers per tile and was slower with one slice: 8,192 tokens of 8 heads of 64,
-  // blocks of 16, 40.7 against 35.4 us.
-  // What bounds it (8,192 tokens, 32 heads of 128, blocks of 32): K/V tiles that feed one head, 3.4 GB
-  // staged of which 2.3 GB miss the L2s; 432 us before the lookahead, the skipped halves and the
-  // fourth workgroup per CU (smaller row caches), now 372 us.  A window of 512 keys, 4,096 tokens of
-  // 32 heads: 67 -> 59 us.
+  // 116, 8,192 tokens 253, now 214; all dense 8,192 tokens 623, now 593).  With slices the CU holds one
+  // workgroup (two with NS = 2), and its loads must run under its own work: K is refilled once every wave
+  // has read it (under the exponentials and the PV product), V after the PV product (under the next QK
+  // product).  That order costs two more barriers per tile and was slower with one slice: 8,192 tokens of
+  // 8 heads of 64, blocks of 16, 40.7 against 35.4 us.
+  // What bounds it: K/V tiles that feed one head.  8,192 tokens, 32 heads of 128, blocks of 32, stage 3.4 GB
+  // (185 us at the rate of the L2-resident staging loop): 270 us, 432 without the lookahead, the skipped
+  // halves, the fourth workgroup per CU and the queues per XCD.  A window of 512 keys, 4,096 tokens of 32
+  // heads: 59 us, 102 without them.
   template <bool LOOK>
   static __device__ __forceinline__ void item(const PrefillArgs& a, int qt, int r, int hs, int b, char* sKV,
                                               float* s_ml, int32_t* s_row, int32_t* s_mask, const Look* lk) {
@@ -1621,8 +1623,9 @@ struct Prefill {
   }
 
   // Item index -> (qt, r, hs, b).  Per lane: v may differ between lanes (the startup reads two
-  // items' offsets in two lanes).  Queued launches: unit order.  Without row_order: query tiles latest first, all rows of a
-  // tile together; with it: row by row (s_row_rank), latest query tiles first within a row.
+  // items' offsets in two lanes).  Queued launches: unit order.  Others: query tiles latest first, all
+  // rows of a tile together, and with row_order the tiles below q_split row by row (s_row_rank), latest
+  // first within a row.
   static __device__ __forceinline__ void decode_item(const PrefillArgs& a, int v, int& qt, int& r, int& hs, int& b) {
     uint32_t rem;
     if constexpr (KS) v = (int)fast_div((uint32_t)v, (uint32_t)a.splits, a.mul_splits);
@@ -2182,10 +2185,9 @@ static int prefill_impl(const char* fn, int dtype,
 
   const int64_t per_tile = (int64_t)a.R * B * a.head_splits;
   const int64_t n_items = (int64_t)a.ntq * per_tile;
-  // Queues: one XCD keeps to a few KV heads, whose K/V its L2 can hold (past the L2s the Infinity Cache
-  // serves 26-30 B/ns per CU, an L2 117-145).  Items that read a whole KV head's rows one head at a time
-  // gain most: 8,192 tokens of 32 heads, blocks of 32, 335 us with one queue, 280 with eight; a window of
-  // 512 175 / 124 us; 32,768 tokens 528 / 449.  Four heads to an item read less: dense 8,192 tokens
+  // Queues: one XCD keeps to a few KV heads, whose K/V its L2 can hold.  Items that read a whole KV head's
+  // rows one head at a time gain most: 8,192 tokens of 32 heads, blocks of 32, 335 us with one queue, 280
+  // with eight; a window of 512 175 / 124 us; 32,768 tokens 528 / 449.  Four heads to an item read less: dense 8,192 tokens
   // 600 / 520, blocks drawn from 8,192 tokens 319 / 315, and past the L2 nothing: the 32K-token prompt (16 MB
   // per head, groups of different densities) 335 / 392 us.  Rows of different lengths turn them off in the
   // kernel (rows_even).

@@ -97,7 +97,9 @@ class _BlockMaskPattern(SparsePattern):
     The CSR depends on the shape only through the block counts (nqb, nkb) and
     the query block offset, so decode steps inside one KV block reuse it; the
     device copies live in a small LRU keyed that way.  The keep ratio is
-    computed from host-side counts, so ``build`` never waits for the GPU.
+    computed from host-side counts: a build that finds its schedule there, or
+    whose mask is made on the CPU, does not wait for the GPU.  A new schedule
+    of the GPU generator reads its rows' entry counts back once.
     """
 
     CACHE_SIZE = 32
