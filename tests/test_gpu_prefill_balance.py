@@ -64,10 +64,10 @@ def _ratio(Hq, rows, B, T, profile, ws_bytes):
     return us[0] / us[1]
 
 
-@pytest.mark.parametrize("B,T", [(1, 8192), (2, 4096)])
+@pytest.mark.parametrize("B,T", [(1, 8192), (2, 4096), (1, 6016)])
 @pytest.mark.parametrize("profile", list(PROFILES))
 def test_one_queue_four_heads(B, T, profile):
-    """Four items per workgroup, the first three dealt by index."""
+    """Four items per workgroup, the first three dealt by index, and three."""
     assert _ratio(32, 8, B, T, profile, int(_lib.load().sa_prefill_workspace_bytes())) <= SLACK
 
 
