@@ -37,7 +37,7 @@
 //    own index and claims further ones from an atomic counter, heaviest query tiles first --
 //    or, where a KV head's K/V fit an L2 and the CSR rows are of about one length, from the counter
 //    of its XCD's queue of KV heads.  One- and two-head workgroups over rows of different lengths
-//    claim every item.
+//    claim every item, from one queue or, where its XCD's holds about its share, from that.
 //
 // MFMA 32x32x16 lane layouts used (l = lane, g = l / 32):
 //   A (32 x 16): lane l holds row l % 32, k = 8g .. 8g+7
@@ -116,7 +116,7 @@ struct PrefillArgs {
   int splits;
   uint32_t mul_splits;
   float* part;
-  // Launches with queues (queues == N_XCD, otherwise 1), if their rows are even: the items in unit order, a unit being what reads
+  // Launches with queues (queues == N_XCD, otherwise 1), if they use them (s_queued): the items in unit order, a unit being what reads
   // the KV heads of one or a few (b, kvh) -- latest query tiles first, then the unit_heads KV heads, the
   // per_head items of each -- cut into one contiguous queue per XCD.  per_unit = ntq * per_qt items,
   // per_qt = unit_heads * per_head, per_head = (R / Hkv) * head_splits.
@@ -168,7 +168,7 @@ __device__ __forceinline__ unsigned long long add_claim(unsigned long long* clai
 constexpr int MAX_ORDERED_ROWS = 256;
 __shared__ int s_row_rank[MAX_ORDERED_ROWS];
 
-// Whether a launch with queues (PrefillArgs::queues) uses them: if its rows are even (rows_even).
+// Whether a launch with queues (PrefillArgs::queues) uses them: rows_even, queues_even.
 __shared__ int s_queued;
 
 // Timeline instantiation (TL) of the persistent four-head loop: shader-clock cycles (s_memtime)
@@ -208,6 +208,30 @@ __device__ __forceinline__ float halves_sum(float x) {
 __device__ __forceinline__ float halves_max(float x) {
   const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1]));
+}
+
+// Lane l's value from lane l ^ 1, l ^ 2, and the mirror images of l in its 8 and 16 lanes.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), CTRL, 0xf, 0xf, true));
+}
+
+// Sum / max of a value over the wave, in every lane, without LDS.
+__device__ __forceinline__ float wave_sum(float x) {
+  x += dpp<0xB1>(x);
+  x += dpp<0x4E>(x);
+  x += dpp<0x141>(x);
+  x += dpp<0x140>(x);
+  const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return halves_sum(__uint_as_float(s[0]) + __uint_as_float(s[1]));
+}
+__device__ __forceinline__ float wave_max(float x) {
+  x = fmaxf(x, dpp<0xB1>(x));
+  x = fmaxf(x, dpp<0x4E>(x));
+  x = fmaxf(x, dpp<0x141>(x));
+  x = fmaxf(x, dpp<0x140>(x));
+  const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return halves_max(fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1])));
 }
 
 __device__ __forceinline__ __attribute__((address_space(3))) void* lds_ptr(const void* p) {
@@ -821,7 +845,7 @@ struct Prefill {
 
   // ---- queues (persistent loop) ---------------------------------------------------------------
   // Queue x holds the items [queue_start(x), queue_start(x + 1)); the workgroups w = x mod queues own
-  // it.  Its first LOOKAHEAD items per owner are dealt, the others claimed, so every item is dealt or
+  // it.  Its first `dealt` items per owner are dealt, the others claimed, so every item is dealt or
   // claimed once: an owner leaves its queue only when the queue has run out.
   enum : int { CL_QUEUE = 0, CL_TAKEN = 1, CL_WORDS = 2 };  // queue claimed from, items taken
   static constexpr bool QUEUES = !KS && !TL && NS == 1;  // slices: at most one item per workgroup
@@ -850,17 +874,42 @@ struct Prefill {
       sum += len;
       longest = fmaxf(longest, len);
     }
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-      sum += __shfl_xor(sum, d);
-      longest = fmaxf(longest, __shfl_xor(longest, d));
-    }
+    sum = wave_sum(sum);
+    longest = wave_max(longest);
     return longest * (float)a.R <= sum * (PIPE ? 1.0625f : 1.25f);
   }
 
+  // Whether no queue of uneven rows holds more than 3/4 (one head to an item) or 1/4 (two) above its share
+  // (none does with every sequence of a batch in a queue of its own).  Queue x holds per_queue heads from
+  // x per_queue on, head h those rows that KV head h mod Hkv's query heads read.  Items claimed one by one,
+  // one queue / a queue per XCD (us), most loaded queue over the mean in brackets: a schedule per head,
+  // 4 x 4,096 tokens of 32 heads, half of the KV heads dense 481 / 392 (1.0), windows of 2 to 30 % 286 / 231
+  // (1.5), 8,192 tokens 223 / 219 (1.7), 240 / 264 (2.2); 16 heads, two to an item, 2 x 8,192 tokens 190 / 175
+  // (1.3), 198 / 214 (1.7).
+  static __device__ __forceinline__ bool queues_even(const PrefillArgs& a) {
+    const int per_queue = a.B * a.Hkv / N_XCD, rest = per_queue % a.Hkv;
+    const int rows_per_kv = a.R == a.Hkv ? 1 : a.heads_per_kv;
+    float sum = 0.f, part[N_XCD] = {};  // of the rows; of those in each queue's `rest` heads
+    for (int r = threadIdx.x & 63; r < a.R; r += 64) {
+      const int32_t* o = a.offsets + r * a.offsets_stride;
+      const float len = (float)(o[a.nqb] - o[0]);
+      sum += len;
+#pragma unroll
+      for (int x = 0; x < N_XCD; ++x) {
+        const int d = r / rows_per_kv - x * per_queue % a.Hkv;
+        if (d + (d < 0 ? a.Hkv : 0) < rest) part[x] += len;
+      }
+    }
+    float longest = 0.f;
+#pragma unroll
+    for (int x = 0; x < N_XCD; ++x) longest = fmaxf(longest, wave_sum(part[x]));
+    sum = wave_sum(sum);
+    return (longest + (float)(per_queue / a.Hkv) * sum) * (float)N_XCD <= sum * (float)a.B * (HW == 1 ? 1.75f : 1.25f);
+  }
+
   // Claim number n of queue x: its item, or n_items where the queue has run out.
-  static __device__ __forceinline__ int queue_item(const PrefillArgs& a, int x, unsigned n, int n_items) {
-    const int s = queue_start(a, x, n_items) + LOOKAHEAD * owners(a);
+  static __device__ __forceinline__ int queue_item(const PrefillArgs& a, int x, unsigned n, int n_items, int dealt) {
+    const int s = queue_start(a, x, n_items) + dealt * owners(a);
     return n < (unsigned)(queue_start(a, x + 1, n_items) - s) ? s + (int)n : n_items;
   }
 
@@ -880,15 +929,17 @@ struct Prefill {
   // Once a queue has run out, each of its owners looks at one of the other seven, by its index (all of
   // them looking at all seven counters costs more than it balances, 1,024 workgroups on 8 lines: 8,192
   // tokens of 32 heads 293 against 280 us, with a window 137 against 124).
-  static __device__ __forceinline__ int queue_claimed(const PrefillArgs& a, int* cl, unsigned n, int n_items) {
+  static __device__ __forceinline__ int queue_claimed(const PrefillArgs& a, int* cl, unsigned n, int n_items,
+                                                      int dealt) {
     const int own = (int)blockIdx.x % N_XCD;
     int x = cl[CL_QUEUE];
-    int v = queue_item(a, x, n, n_items);
+    int v = queue_item(a, x, n, n_items, dealt);
     if (v >= n_items && x == own) {
       x = (own + 1 + (int)(blockIdx.x / N_XCD) % (N_XCD - 1)) % N_XCD;
       unsigned long long* c = &a.claims[x * WS_QUEUE + WS_CLAIMS];
-      if (queue_item(a, x, (unsigned)__hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), n_items) < n_items) {
-        v = queue_item(a, x, (unsigned)atomicAdd(c, 1ull), n_items);
+      if (queue_item(a, x, (unsigned)__hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), n_items, dealt) <
+          n_items) {
+        v = queue_item(a, x, (unsigned)atomicAdd(c, 1ull), n_items, dealt);
         cl[CL_QUEUE] = x;
       }
     }
@@ -984,7 +1035,7 @@ struct Prefill {
       lk.meta2[6] = ld.b2;
       int v3 = lk.n_items;
       if (lk.taken)
-        v3 = queued(a) ? queue_claimed(a, lk.cl, (unsigned)ld.nv, lk.n_items)
+        v3 = queued(a) ? queue_claimed(a, lk.cl, (unsigned)ld.nv, lk.n_items, LOOKAHEAD)
                        : claimed_item(a.claims, a.status, ld.nv, lk.taken, lk.fixed, lk.n_items);
       lk.vid3[0] = v3;
     }
@@ -1815,10 +1866,16 @@ struct Prefill {
   }
 
   // Items one at a time: the workgroup's only one (no workspace), or, for one- and two-head workgroups
-  // over uneven rows, one queue of which every item is claimed when the one before it has ended.
+  // over uneven rows, every item is claimed when the one before it has ended, from one queue or, if those
+  // are even, from a queue per XCD.
   static constexpr bool CLAIM_EACH = QUEUES && !PIPE;
   static __device__ __forceinline__ void run_items(const PrefillArgs& a, int n_items, char* sKV, char* sQ, float* s_ml,
                                                    int32_t* s_row, int32_t* s_mask) {
+    __shared__ int s_cl[CL_WORDS];
+    if (CLAIM_EACH && threadIdx.x == 0) {
+      s_cl[CL_QUEUE] = (int)blockIdx.x % N_XCD;
+      s_cl[CL_TAKEN] = 0;
+    }
     for (int taken = 0;; taken = 1) {
       int v;
       if (!CLAIM_EACH || !a.claims) {
@@ -1831,7 +1888,10 @@ struct Prefill {
         v = ((seq / chunk) * N_XCD + xcd) * chunk + seq % chunk;
       } else {
         __shared__ int s_item;
-        if (threadIdx.x == 0) s_item = claimed_item(a.claims, a.status, add_claim(a.claims, taken), taken, 0, n_items);
+        if (threadIdx.x == 0)
+          s_item = queued(a) ? queue_claimed(a, s_cl, (unsigned)atomicAdd(&a.claims[s_cl[CL_QUEUE] * WS_QUEUE + WS_CLAIMS], 1ull),
+                                             n_items, 0)
+                             : claimed_item(a.claims, a.status, add_claim(a.claims, taken), taken, 0, n_items);
         __syncthreads();
         v = s_item;
         __syncthreads();
@@ -1870,8 +1930,9 @@ struct Prefill {
       // windows of 1 to 12 blocks 41 against 55).
       const bool queues = QUEUES && a.queues > 1;
       const bool even = queues || (CLAIM_EACH && n_items > 2 * (int)gridDim.x) ? rows_even(a) : true;
-      if (queues && threadIdx.x == 0) s_queued = even;
-      if (a.row_order && !(queues && even)) rank_rows(a, reinterpret_cast<int*>(sKV));  // K/V buffers are free here
+      const bool use = queues && (even || (CLAIM_EACH && queues_even(a)));
+      if (queues && threadIdx.x == 0) s_queued = use;
+      if (a.row_order && !use) rank_rows(a, reinterpret_cast<int*>(sKV));  // K/V buffers are free here
       if (CLAIM_EACH && !even) {
         __syncthreads();  // the ranks are visible
         dealt = false;
