@@ -503,8 +503,8 @@ struct Prefill {
 
   // Work item (qt, r, hs, b) whose CSR row holds entries [e0, e0 + n_ent): pointers and
   // positions only, no memory reads.
-  static __device__ __forceinline__ Item setup_base(const PrefillArgs& a, int qt, int r, int hs, int b, int e0,
-                                                    int n_ent) {
+  static __device__ __forceinline__ Item setup(const PrefillArgs& a, int qt, int r, int hs, int b, int e0,
+                                               int n_ent) {
     Item it;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -531,16 +531,16 @@ struct Prefill {
     return it;
   }
 
-  // Sets up work item (qt, r, hs, b): query tile qt (64 rows) of CSR row r, batch b, head
+  // Sets up work item (qt, r, hs, b) without lookahead: query tile qt (64 rows) of CSR row r, batch b, head
   // split hs.  Each wave owns 32 rows (half hf) of one query head; every K/V tile staged in
   // LDS feeds all NW waves.  Caches the CSR row of the query tile in s_row (callers barrier
   // before, so no wave still reads it).
-  static __device__ __forceinline__ Item setup(const PrefillArgs& a, int qt, int r, int hs, int b, int32_t* s_row,
-                                               int32_t* s_mask) {
+  static __device__ __forceinline__ Item setup_row(const PrefillArgs& a, int qt, int r, int hs, int b, int32_t* s_row,
+                                                   int32_t* s_mask) {
     // CSR row of this query tile; each block holds 2^tpb_log2 key tiles.
     const int32_t* offs = a.offsets + r * a.offsets_stride + (qt >> a.qpb_log2);
     const int e0 = offs[0];
-    const Item it = setup_base(a, qt, r, hs, b, e0, offs[1] - e0);
+    const Item it = setup(a, qt, r, hs, b, e0, offs[1] - e0);
     if (it.cached) {
       const int n_ent = it.n_tiles >> a.tpb_log2;
       for (int x = threadIdx.x; x < n_ent; x += NT) s_row[x] = it.prow[e0 + x];
@@ -866,9 +866,18 @@ struct Prefill {
   // one dense KV head of eight, r = 5.2, 212 / 405.  One head to an item, 8,192 tokens of 32 heads, every
   // item claimed when the last has ended / three dealt and a queue per XCD: r = 1.2 216 / 200, 1.4 218 / 220,
   // 1.7 223 / 270, 5.2 274 / 545.
-  static __device__ __forceinline__ bool rows_even(const PrefillArgs& a) {
-    float sum = 0.f, longest = 0.f;
-    for (int r = threadIdx.x & 63; r < a.R; r += 64) {
+  struct RowEnds {
+    int32_t first, end;  // of lane r's row
+  };
+  static __device__ __forceinline__ RowEnds row_ends(const PrefillArgs& a) {
+    const int r = threadIdx.x & 63;
+    if (r >= a.R) return RowEnds{0, 0};
+    const int32_t* o = a.offsets + r * a.offsets_stride;
+    return RowEnds{o[0], o[a.nqb]};
+  }
+  static __device__ __forceinline__ bool rows_even(const PrefillArgs& a, const RowEnds& ends) {
+    float sum = (float)(ends.end - ends.first), longest = sum;
+    for (int r = 64 + (threadIdx.x & 63); r < a.R; r += 64) {
       const int32_t* o = a.offsets + r * a.offsets_stride;
       const float len = (float)(o[a.nqb] - o[0]);
       sum += len;
@@ -1119,9 +1128,8 @@ struct Prefill {
   // (185 us at the rate of the L2-resident staging loop): 270 us, 432 without the lookahead, the skipped
   // halves, the fourth workgroup per CU and the queues per XCD.  A window of 512 keys, 4,096 tokens of 32
   // heads: 59 us, 102 without them.
-  template <bool LOOK>
   static __device__ __forceinline__ void item(const PrefillArgs& a, int qt, int r, int hs, int b, char* sKV,
-                                              float* s_ml, int32_t* s_row, int32_t* s_mask, const Look* lk) {
+                                              float* s_ml, int32_t* s_row, int32_t* s_mask, const Look& lk) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int slice = NS == 1 ? 0 : wave / TW;
@@ -1134,7 +1142,7 @@ struct Prefill {
       sK = sKV + buf * 2 * TILE_BYTES;
       sV = sK + TILE_BYTES;
     };
-    const Item it = LOOK ? setup_base(a, qt, r, hs, b, lk->e0, lk->n_ent) : setup(a, qt, r, hs, b, s_row, s_mask);
+    const Item it = setup(a, qt, r, hs, b, lk.e0, lk.n_ent);
     // Q^T as the B operand of S^T = K Q^T: lane holds row l32, d = 16c + 8g .. +7.
     u32x4 qf[D / 16];
     {
@@ -1190,14 +1198,10 @@ struct Prefill {
     }
     // One wait for the first tiles and the lookahead's reads (and Q: with a load pending at the
     // loop's entry the compiler would wait for every load in each step).
-    if constexpr (LOOK) {
-      LookLoads ld;
-      look_issue(a, *lk, ld);
-      wait_dma();
-      look_commit(a, *lk, ld);
-    } else {
-      wait_dma();
-    }
+    LookLoads ld;
+    look_issue(a, lk, ld);
+    wait_dma();
+    look_commit(a, lk, ld);
     if (!any) __syncthreads();  // the lookahead's writes are visible (else by the first step's barrier)
 
     // S^T = K Q^T of the tile: two independent accumulation chains keep the matrix pipe busy.
@@ -1358,7 +1362,7 @@ struct Prefill {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     tl_stamp(TL_GAP);
-    const Item it = LOOK ? setup_base(a, qt, r, hs, b, lk->e0, lk->n_ent) : setup(a, qt, r, hs, b, s_row, s_mask);
+    const Item it = LOOK ? setup(a, qt, r, hs, b, lk->e0, lk->n_ent) : setup_row(a, qt, r, hs, b, s_row, s_mask);
     char* sQw = sQ + wave * WAVE_BYTES;
     load_q(a, it.qb, it.q_row0, sQw, lane);  // Q^T operand of this wave into LDS
     tl_stamp(TL_SETUP_Q);
@@ -1746,53 +1750,18 @@ struct Prefill {
     b = __builtin_amdgcn_readfirstlane(b);
   }
 
-  static __device__ __forceinline__ void process(const PrefillArgs& a, int v, char* sKV, char* sQ, float* s_ml,
-                                                 int32_t* s_row, int32_t* s_mask) {
-    int qt, r, hs, b;
-    decode_item_uniform(a, v, qt, r, hs, b);
-    if constexpr (PIPE)
-    {
-      int vb_first = 0;
-      item_pipelined<false>(a, qt, r, hs, b, sKV, sQ, s_row, s_mask, nullptr, vb_first, v);
-    }
-    else
-      item<false>(a, qt, r, hs, b, sKV, s_ml, s_row, s_mask, nullptr);
+  static constexpr bool CLAIM_EACH = QUEUES && !PIPE;
+
+  // Thread 0: the next item of a workgroup that claims each when it has ended the last, from one queue
+  // (`taken` since the last claim) or a queue per XCD, or n_items.
+  static __device__ __forceinline__ int claim_item(const PrefillArgs& a, int n_items, int taken, int* cl) {
+    if (!queued(a)) return claimed_item(a.claims, a.status, add_claim(a.claims, taken), taken, 0, n_items);
+    return queue_claimed(a, cl, (unsigned)atomicAdd(&a.claims[cl[CL_QUEUE] * WS_QUEUE + WS_CLAIMS], 1ull), n_items, 0);
   }
 
-  // Persistent loop with lookahead.  The first LOOKAHEAD items of a workgroup w (of g) are fixed by w:
-  // w, 2g - 1 - w and 2g + w, so that the workgroup with the lightest first item takes the heaviest
-  // second one; later ones are claimed from the counter.  Four-head launches that have no later ones run
-  // the third round in reverse too: g is a multiple of the rows, and 2g + w is of the first item's row
-  // (6,016 tokens of 32 heads, one dense KV head of eight: 183 us with 2g + w, 145 with 3g - 1 - w).  (Claimed ahead, the first ones all went to the
-  // workgroups that started first, three each: 128 items of 64-79 tiles -- 1,000 queries of 32 heads on
-  // 5,000 keys -- ran on 43 CUs, 297 us; one item per workgroup takes 107 us.  Three neighbours, 3w to
-  // 3w + 2, give a few workgroups the longest three: four items per workgroup, dense 8,192 tokens of 32
-  // heads 711 us against 581; one dense KV head among eight of five blocks 498 against 208; six per
-  // workgroup, dense 12,288 tokens 1,266 against 1,218; the 32K-token prompt, 16 per workgroup, the same.)
-  // Item i of this workgroup finds in LDS its id,
-  // CSR offsets and (qt, r, hs, b) (slot i % 4 of s_meta) and its row (row cache i % 2), and
-  // the id, offsets and row of item i + 1 and the id of item i + 2; its prologue fetches the
-  // row of item i + 1, the offsets and (qt, r, hs, b) of item i + 2 and claims item i + 3
-  // (Look).  The ids after one past the end are past it too, so the first such id ends the loop, in
-  // every wave at once.
-  static __device__ __forceinline__ void run_lookahead(const PrefillArgs& a, int n_items, char* sKV, char* sQ,
-                                                       float* s_ml, int32_t* s_row, int32_t* s_mask) {
-    int vb_first = 0;  // V buffer free for the next item's first tile
-    // Per slot k = item index mod 4: id, CSR offsets (first, end) and (qt, r, hs, b); the loop
-    // top reads an item's whole slot (and the ids and offsets of the next two) in one batch.
-    __shared__ __attribute__((aligned(16))) int s_meta[4][8];
+  // Offsets and (qt, r, hs, b) of the items in slots 0 and 1; no barrier after it.
+  static __device__ __forceinline__ void first_offsets(const PrefillArgs& a, int n_items, int (*s_meta)[8]) {
     const int tid = threadIdx.x;
-    __shared__ int s_cl[CL_WORDS];
-    if (tid == 0) {
-      const int x = queued(a) ? (int)blockIdx.x % N_XCD : 0, g = owners(a);
-      const int w = queued(a) ? (int)blockIdx.x / N_XCD : (int)blockIdx.x;
-      const int s = queue_start(a, x, n_items);
-      s_meta[0][0] = s + w;
-      s_meta[1][0] = s + 2 * g - 1 - w;
-      s_meta[2][0] = s + (PIPE && n_items <= LOOKAHEAD * g ? 3 * g - 1 - w : 2 * g + w);
-      s_cl[CL_QUEUE] = x;
-      s_cl[CL_TAKEN] = LOOKAHEAD;
-    }
     __syncthreads();
     if (tid < 2) {
       const int v = s_meta[tid][0];
@@ -1808,8 +1777,99 @@ struct Prefill {
         s_meta[tid][6] = b;
       }
     }
-    __syncthreads();
-    {
+  }
+
+  // The item of a workgroup without a workspace (past the end: padding of the last round).  Consecutive
+  // workgroups go to the 8 XCDs in turn; chunks of XCD_CHUNK consecutive query tiles (all rows) are dealt
+  // to the XCDs round-robin so every XCD gets an even share of each row's work, while neighbouring tiles
+  // (which share window and global key blocks) stay in one XCD's L2.
+  static __device__ __forceinline__ int only_item(const PrefillArgs& a) {
+    const int per_tile = a.R * a.B * a.head_splits;
+    const int chunk = XCD_CHUNK * per_tile;
+    const int xcd = blockIdx.x % N_XCD, seq = blockIdx.x / N_XCD;
+    return ((seq / chunk) * N_XCD + xcd) * chunk + seq % chunk;
+  }
+
+  // The dealt items' ids -- without a workspace (smaller workgroups) the only one -- and the first two's
+  // offsets.
+  static __device__ __forceinline__ void deal(const PrefillArgs& a, int n_items, int (*s_meta)[8], int* s_cl) {
+    if (!PIPE && threadIdx.x == 0 && !a.claims) {
+      s_meta[0][0] = only_item(a);
+      s_meta[1][0] = n_items;
+      s_meta[2][0] = n_items;
+    } else if (threadIdx.x == 0) {
+      const int x = queued(a) ? (int)blockIdx.x % N_XCD : 0, g = owners(a);
+      const int w = queued(a) ? (int)blockIdx.x / N_XCD : (int)blockIdx.x;
+      const int s = queue_start(a, x, n_items);
+      s_meta[0][0] = s + w;
+      s_meta[1][0] = s + 2 * g - 1 - w;
+      s_meta[2][0] = s + (PIPE && n_items <= LOOKAHEAD * g ? 3 * g - 1 - w : 2 * g + w);
+      s_cl[CL_QUEUE] = x;
+      s_cl[CL_TAKEN] = LOOKAHEAD;
+    }
+    first_offsets(a, n_items, s_meta);
+  }
+
+  // The items of a workgroup, one after another: dealt and claimed ahead (with lookahead), or each claimed
+  // when the last has ended.  Dealt: the first LOOKAHEAD items of a workgroup w (of g) are fixed by w:
+  // w, 2g - 1 - w and 2g + w, so that the workgroup with the lightest first item takes the heaviest
+  // second one; later ones are claimed from the counter.  Four-head launches that have no later ones run
+  // the third round in reverse too: g is a multiple of the rows, and 2g + w is of the first item's row
+  // (6,016 tokens of 32 heads, one dense KV head of eight: 183 us with 2g + w, 145 with 3g - 1 - w).
+  // (Claimed ahead, the first ones all went to the workgroups that started first, three each: 128 items of
+  // 64-79 tiles -- 1,000 queries of 32 heads on 5,000 keys -- ran on 43 CUs, 297 us; one item per workgroup
+  // takes 107 us.  Three neighbours, 3w to 3w + 2, give a few workgroups the longest three: four items per
+  // workgroup, dense 8,192 tokens of 32 heads 711 us against 581; one dense KV head among eight of five
+  // blocks 498 against 208; six per workgroup, dense 12,288 tokens 1,266 against 1,218; the 32K-token
+  // prompt, 16 per workgroup, the same.)
+  // Item i of this workgroup finds in LDS its id, CSR offsets and (qt, r, hs, b) (slot i % 4 of s_meta) and
+  // its row (row cache i % 2), and the id, offsets and row of item i + 1 and the id of item i + 2; its
+  // prologue fetches the row of item i + 1, the offsets and (qt, r, hs, b) of item i + 2 and claims item
+  // i + 3 (Look).  The ids after one past the end are past it too, so the first such id ends the loop, in
+  // every wave at once.
+  // Returns whether the items were dealt and claimed ahead.
+  static __device__ __forceinline__ bool run_items(const PrefillArgs& a, int n_items, char* sKV, char* sQ, float* s_ml,
+                                                   int32_t* s_row, int32_t* s_mask) {
+    int vb_first = 0;  // V buffer free for the next item's first tile
+    // Per slot k = item index mod 4: id, CSR offsets (first, end) and (qt, r, hs, b); the loop
+    // top reads an item's whole slot (and the ids and offsets of the next two) in one batch.
+    __shared__ __attribute__((aligned(16))) int s_meta[4][8];
+    const int tid = threadIdx.x;
+    __shared__ int s_cl[CL_WORDS];
+    // Queues and dealt items are for even rows (rows_even).  Smaller workgroups are dealt their items while
+    // the rows' lengths are read, and claim every item if the rows turn out uneven.  Up to two items per
+    // workgroup the second round, which runs in reverse, balances uneven rows as well as claims do (2 x
+    // 4,096 tokens of 16 heads, one dense KV head of eight: 118 us dealt, 112 claimed; windows of 1 to 12
+    // blocks 41 against 55).
+    const bool queues = QUEUES && a.queues > 1;
+    bool each = false;  // every item is claimed when the last has ended
+    int* s_len = reinterpret_cast<int*>(sKV);  // the K/V buffers are free here
+    if constexpr (PIPE) {
+      const bool even = queues ? rows_even(a, row_ends(a)) : true;
+      if (queues && tid == 0) s_queued = even;
+      if (a.row_order && !(queues && even)) rank_rows(a, s_len);
+      deal(a, n_items, s_meta, s_cl);
+    } else {
+      const bool check = a.claims && (queues || (CLAIM_EACH && n_items > 2 * (int)gridDim.x));
+      RowEnds ends{0, 0};
+      if (check) ends = row_ends(a);
+      if (queues && tid == 0) s_queued = 1;
+      if (a.row_order && !queues) rank_rows(a, s_len);
+      deal(a, n_items, s_meta, s_cl);
+      if (CLAIM_EACH && check && !rows_even(a, ends)) {
+        each = true;
+        const bool use = queues && queues_even(a);
+        __syncthreads();  // every wave has read s_queued and the ranks
+        if (queues && a.row_order && !use) rank_rows(a, s_len);
+        if (tid == 0) {
+          s_queued = use;
+          s_cl[CL_QUEUE] = (int)blockIdx.x % N_XCD;
+          s_cl[CL_TAKEN] = 0;
+        }
+      }
+    }
+    auto first_row = [&] {  // of the item in slot 0
+      __syncthreads();
       const int v = s_meta[0][0];
       const int e0 = s_meta[0][1], n = s_meta[0][2] - e0;
       if (v < n_items && n <= RC) {
@@ -1819,9 +1879,21 @@ struct Prefill {
           if (SUB) s_mask[x] = a.tile_masks[r * a.masks_stride + e0 + x];
         }
       }
-    }
-    __syncthreads();  // publishes the row cache of item 0
-    for (int i = 0;; ++i) {
+      __syncthreads();  // publishes the row cache of item 0
+    };
+    if (!each) first_row();
+    for (int i = 0, taken = 0;; ++i) {
+      if (CLAIM_EACH && each) {  // as a first item, with none after it
+        i = 0;
+        if (tid == 0) {
+          s_meta[0][0] = claim_item(a, n_items, taken, s_cl);
+          s_meta[1][0] = n_items;
+          s_meta[2][0] = n_items;
+        }
+        taken = 1;
+        first_offsets(a, n_items, s_meta);
+        first_row();
+      }
       tl_stamp(TL_LOOP_TOP);
       // The metadata of item i was published by item i - 1's barriers; the K/V buffers are
       // freed by the barrier in the item's prologue.  Values read from LDS are the same in
@@ -1861,45 +1933,9 @@ struct Prefill {
       if constexpr (PIPE)
         item_pipelined<true>(a, qt, r, hs, b, sKV, sQ, row, mask, &lk, vb_first, v);
       else
-        item<true>(a, qt, r, hs, b, sKV, s_ml, row, mask, &lk);
+        item(a, qt, r, hs, b, sKV, s_ml, row, mask, lk);
     }
-  }
-
-  // Items one at a time: the workgroup's only one (no workspace), or, for one- and two-head workgroups
-  // over uneven rows, every item is claimed when the one before it has ended, from one queue or, if those
-  // are even, from a queue per XCD.
-  static constexpr bool CLAIM_EACH = QUEUES && !PIPE;
-  static __device__ __forceinline__ void run_items(const PrefillArgs& a, int n_items, char* sKV, char* sQ, float* s_ml,
-                                                   int32_t* s_row, int32_t* s_mask) {
-    __shared__ int s_cl[CL_WORDS];
-    if (CLAIM_EACH && threadIdx.x == 0) {
-      s_cl[CL_QUEUE] = (int)blockIdx.x % N_XCD;
-      s_cl[CL_TAKEN] = 0;
-    }
-    for (int taken = 0;; taken = 1) {
-      int v;
-      if (!CLAIM_EACH || !a.claims) {
-        // Consecutive workgroups go to the 8 XCDs in turn; chunks of XCD_CHUNK consecutive query tiles
-        // (all rows) are dealt to the XCDs round-robin so every XCD gets an even share of each row's
-        // work, while neighbouring tiles (which share window and global key blocks) stay in one XCD's L2.
-        const int per_tile = a.R * a.B * a.head_splits;
-        const int chunk = XCD_CHUNK * per_tile;
-        const int xcd = blockIdx.x % N_XCD, seq = blockIdx.x / N_XCD;
-        v = ((seq / chunk) * N_XCD + xcd) * chunk + seq % chunk;
-      } else {
-        __shared__ int s_item;
-        if (threadIdx.x == 0)
-          s_item = queued(a) ? queue_claimed(a, s_cl, (unsigned)atomicAdd(&a.claims[s_cl[CL_QUEUE] * WS_QUEUE + WS_CLAIMS], 1ull),
-                                             n_items, 0)
-                             : claimed_item(a.claims, a.status, add_claim(a.claims, taken), taken, 0, n_items);
-        __syncthreads();
-        v = s_item;
-        __syncthreads();
-      }
-      if (v >= n_items) break;  // none left, or a padding workgroup of the last round
-      process(a, v, sKV, sQ, s_ml, s_row, s_mask);
-      if (!CLAIM_EACH || !a.claims) break;
-    }
+    return !each;
   }
 
   static __device__ void run(const PrefillArgs& a) {
@@ -1911,6 +1947,19 @@ struct Prefill {
     __shared__ int32_t s_mask[SUB ? 2 * RC : 1];  // sub-block masks of the cached rows
     const int n_items = a.ntq * a.R * a.B * a.head_splits * (KS ? a.splits : 1);
 
+    // Four-head workgroups have an instance of their item for launches without a workspace: with one item
+    // for both, launches of few items took 2-6 % longer (32,768 tokens the same).
+    if constexpr (PIPE) {
+      if (!a.claims) {
+        const int v = only_item(a);
+        if (v >= n_items) return;
+        int qt, r, hs, b;
+        decode_item_uniform(a, v, qt, r, hs, b);
+        int vb_first = 0;
+        item_pipelined<false>(a, qt, r, hs, b, sKV, sQ, s_row, s_mask, nullptr, vb_first, v);
+        return;
+      }
+    }
     unsigned long long* rec = nullptr;  // TL: this workgroup's record
     if constexpr (TL) {
       rec = a.timeline + (int64_t)blockIdx.x * TL_WORDS;
@@ -1923,34 +1972,13 @@ struct Prefill {
       const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
       if (wave % HW == 0 && (threadIdx.x & 63) == 0) s_tl[wave / HW][TL_NOW] = (unsigned)__builtin_amdgcn_s_memtime();
     }
-    bool dealt = a.claims;
-    if (dealt) {
-      // Up to two items per workgroup the second round, which runs in reverse, balances uneven rows as well
-      // as claims do (2 x 4,096 tokens of 16 heads, one dense KV head of eight: 118 us dealt, 112 claimed;
-      // windows of 1 to 12 blocks 41 against 55).
-      const bool queues = QUEUES && a.queues > 1;
-      const bool even = queues || (CLAIM_EACH && n_items > 2 * (int)gridDim.x) ? rows_even(a) : true;
-      const bool use = queues && (even || (CLAIM_EACH && queues_even(a)));
-      if (queues && threadIdx.x == 0) s_queued = use;
-      if (a.row_order && !use) rank_rows(a, reinterpret_cast<int*>(sKV));  // K/V buffers are free here
-      if (CLAIM_EACH && !even) {
-        __syncthreads();  // the ranks are visible
-        dealt = false;
-      }
-    }
-    if (!dealt) {
-      run_items(a, n_items, sKV, sQ, s_ml, s_row, s_mask);
-      return;
-    }
-
-    // Persistent: the dealt items, then claims until one fails.
     const int fixed = LOOKAHEAD * (int)gridDim.x;
     // All items dealt: no workgroup claims, and one looks whether the claims word was zero (read
     // here, looked at after its items, so nothing waits for it).
     unsigned long long seen = 0;
-    if (n_items <= fixed && blockIdx.x == 0 && threadIdx.x == 0)
+    if (a.claims && n_items <= fixed && blockIdx.x == 0 && threadIdx.x == 0)
       seen = __hip_atomic_load(a.claims, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    run_lookahead(a, n_items, sKV, sQ, s_ml, s_row, s_mask);
+    const bool dealt = run_items(a, n_items, sKV, sQ, s_ml, s_row, s_mask);
     if constexpr (TL) {
       __syncthreads();  // every stamp is in LDS
       if (threadIdx.x == 0) {
@@ -1959,7 +1987,7 @@ struct Prefill {
       }
       if (threadIdx.x < 2 * TL_HALF_WORDS) rec[4 + threadIdx.x] = s_tl[threadIdx.x / TL_HALF_WORDS][threadIdx.x % TL_HALF_WORDS];
     }
-    if (seen != 0) {
+    if (dealt && seen != 0) {
       atomicExch(a.claims, 0ull);
       atomicOr(a.status, WS_SKIPPED);
     }
